@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libamaru_hip.so")
 BUILD = os.path.join(HERE, "_build")
-SOURCES = ["api.hip", "kernels_elem.hip", "kernels_solve.hip", "coarse.hip", "recovery.hip",
+SOURCES = ["api.hip", "kernels_elem.hip", "kernels_solve.hip", "coarse.hip", "matrix_free.hip", "recovery.hip",
            "mesh_gen.hip", "loads.hip", "pattern.hip", "model_build.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-ffp-contract=off",

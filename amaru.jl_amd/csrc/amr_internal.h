@@ -225,6 +225,15 @@ struct amr_model {
     // element tilings (index into the shape's table; -1: the tuned or default one)
     int ke_var = -1, up_var = -1;
     int ke_path = AMR_KE_EXACT;   // element stiffness of the NR iterations (amr_set_ke_path)
+    // matrix-free operator of the PCG (matrix_free.hip): element data in groups
+    // of 16 elements; usable (mf_ok) for all-elastic models without a bad
+    // element, while K is a plain assembly (mf_plain)
+    bool mf_ok = false, mf_plain = false;
+    int64_t mf_ngrp = 0;
+    double *mf_tab = nullptr, *mf_geo = nullptr, *mf_lm = nullptr, *mf_f = nullptr;
+    int32_t *mf_conn = nullptr, *mf_src = nullptr, *mf_flag = nullptr;
+    char *mf_block = nullptr;       // the arrays above are slices of it
+    std::vector<double> mf_tab_h;   // host copy of mf_tab while it is uploaded
 };
 
 enum { SV_UEX = 0, SV_FEX, SV_U, SV_F, SV_DFEX, SV_R, SV_RC, SV_DUA, SV_DUI, SV_DFIN, SV_DUT, SV_X };
@@ -274,6 +283,11 @@ int amr_staging_reserve(AmrStaging &s, hipStream_t st, size_t bytes);  // waits 
 int amr_batch_mount_K(amr_model *const *ms, int n, hipStream_t s, AmrStaging &stg);
 int amr_batch_update(amr_model *const *ms, const double *const *dU, double *const *dFin, int n, hipStream_t s,
                      AmrStaging &stg);
+
+// matrix-free operator (matrix_free.hip)
+int amr_mf_build(amr_model *m, const double *dNdR_host);
+int amr_mf_check(amr_model *m);
+void amr_mf_free(amr_model *m);
 
 // two-level coarse space (coarse.hip): the index structures are built on
 // first use (host work, one wait); Kc^-1 is formed again when

@@ -386,6 +386,7 @@ static void free_model(amr_model *m)
     amr_coarse_free(m);
     amr_recovery_free(m);
     if (m->own_stream) (void)hipStreamSynchronize(m->own_stream);
+    amr_mf_free(m);
     void *ptrs[] = {m->X,    m->conn, m->emat, m->mats,  m->dNdR, m->wip,  m->st_cur, m->st_com, m->Ke,
                     m->rowptr, m->col, m->diag, m->cptr,  m->csrc, m->fptr, m->fsrc,   m->Kv,     m->Kv32,
                     m->Kflag, m->dinv, m->dinv32, m->mask, m->eqd,  m->dF,   m->estat,  m->err,    m->part,
@@ -643,7 +644,9 @@ extern "C" int amr_model_create(amr_model **out, int device, int etype, int nips
     AMR_HIP(hipMemsetAsync(m->st_com, 0, sizeof(double) * AMR_NSTATE * m->nip_total, s));
     AMR_HIP(hipMemsetAsync(m->scal, 0, sizeof(double) * 64, s));
     AMR_HIP(hipMemsetAsync(m->err, 0, 4 * sizeof(int32_t), s));
+    TRY(amr_mf_build(m.get(), dNdR.data()));
     TRY(upload_dofs(m.get(), eq_id, ndofs, nu));
+    TRY(amr_mf_check(m.get()));
     TRY(stage_alloc(m.get()));
     *out = m.release();
     return AMR_OK;

@@ -1299,6 +1299,7 @@ int amr_elem_tiles_tune(amr_model *m, int *ach, int *epw)
 int amr_launch_assemble(amr_model *m, bool flags)
 {
     m->k_version++;
+    m->mf_plain = true;
     if (m->pat.nblk == 0) return AMR_OK;
     unsigned grid = (unsigned)((m->pat.nblk + 255) / 256);
     hipLaunchKernelGGL(assemble_kernel, dim3(grid), dim3(256), 0, m->stream, m->pat.nblk, m->cptr, m->csrc, m->Ke,
@@ -1318,6 +1319,7 @@ int amr_launch_assemble(amr_model *m, bool flags)
 int amr_launch_combine_km(amr_model *m, double a, double b)
 {
     m->k_version++;
+    m->mf_plain = false;
     if (m->pat.nblk == 0) return AMR_OK;
     const unsigned grid = (unsigned)((m->pat.nblk + 255) / 256);
     hipLaunchKernelGGL(combine_km_kernel, dim3(grid), dim3(256), 0, m->stream, m->pat.nblk, a, b, m->Kv, m->Kv32,
@@ -1337,6 +1339,7 @@ int amr_launch_combine_km(amr_model *m, double a, double b)
 int amr_launch_combine_kk(amr_model *m, double a1, const double *K1, double a2)
 {
     m->k_version++;
+    m->mf_plain = false;
     if (m->pat.nblk == 0) return AMR_OK;
     const unsigned grid = (unsigned)((m->pat.nblk + 255) / 256);
     hipLaunchKernelGGL(combine_kk_kernel, dim3(grid), dim3(256), 0, m->stream, m->pat.nblk, a1, K1, a2, m->Kv,
@@ -1761,7 +1764,10 @@ int amr_batch_mount_K(amr_model *const *ms, int n, hipStream_t s, AmrStaging &st
                            ds(bj.o_st), bj.n);
         AMR_HIP(hipGetLastError());
     }
-    for (int j = 0; j < n; j++) ms[j]->k_version++;
+    for (int j = 0; j < n; j++) {
+        ms[j]->k_version++;
+        ms[j]->mf_plain = true;
+    }
     return AMR_OK;
 }
 

@@ -50,15 +50,18 @@ constexpr int MAX_GR = 8192, MAX_GV = 1024;
 
 // scalar and control slots of one model: S_NSCAL doubles, then C_NCTL ints
 // S_RZP0/1: r.z published per parity slot (the sum of that slot's partials)
-enum { S_RZ = 0, S_RR, S_BB, S_THR, S_KX, S_RES, S_ERRN, S_ERRD, S_GAP, S_RZP0, S_RZP1, S_NSCAL = 16 };
+// S_BETA: the running iteration's beta (matrix-free members)
+enum { S_RZ = 0, S_RR, S_BB, S_THR, S_KX, S_RES, S_ERRN, S_ERRD, S_GAP, S_RZP0, S_RZP1, S_BETA, S_NSCAL = 16 };
 __device__ inline int rz_pub(int slot) { return slot ? S_RZP1 : S_RZP0; }
 // C_DONE is read by every workgroup at kernel entry and written only where
 // all workgroups of the model in the running launch agree on it
 // (breakdown); the convergence test writes C_STOP, which the next SpMV
 // promotes to C_DONE, so no workgroup ever sees a flag raised during its
 // own launch.  C_ITERS is advanced by the SpMV's first tile and read by the
-// kernels after it.
-enum { C_DONE = 0, C_ITERS, C_BREAK, C_NAN, C_STOP, C_NCTL = 16 };
+// kernels after it.  C_PREV is the number of completed iterations, advanced
+// by the update kernel: the matrix-free operator's tiles read it (one of them
+// writes C_ITERS in the same launch).
+enum { C_DONE = 0, C_ITERS, C_BREAK, C_NAN, C_STOP, C_PREV, C_NCTL = 16 };
 constexpr int SEG_DBL = 32;  // doubles per model in a pool's scalar array
 static_assert(S_NSCAL + C_NCTL / 2 <= SEG_DBL, "scalar block");
 // partial buffers inside m->part
@@ -152,6 +155,16 @@ struct SegDesc {
     const int32_t *agg, *aggptr, *aggnodes;
     const double *cent, *X, *Kinv;
     double *cvec, *yvec;
+    // matrix-free operator (null geo: the assembled matrix): element data of
+    // matrix_free.hip, tiles of 4 mfG groups of 16 elements, and the map
+    // node -> element products (CSR over nodes)
+    const double *geo, *lm, *tab;
+    const int32_t *mfconn, *fptr, *mfsrc;
+    double *mff;
+    int64_t ngrp;
+    int mfG;
+    int npq;                      // partials of p.q
+    int fuse;                     // p = z + beta p formed by the operator and update kernels
 };
 
 // r.z with z = M r: the Jacobi part's partials plus, two-level, the coarse
@@ -617,32 +630,237 @@ __global__ void __launch_bounds__(WGS) pcg_spmv_kernel(const SegDesc *__restrict
     }
 }
 
-__global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl)
+// ------------------------------------------------- matrix-free operator
+//
+// f_e = Be' (coef De) Be p_e for the elements of a tile and the tile's partial
+// of p.q = sum_e p_e . f_e (p is 0 at prescribed dofs); pcg_update sums the f_e
+// of each node into q.  One wave per group of 16 elements (lane l = 16 g + c:
+// element c, node slots 4 s + g, IP slots 4 k + g; see matrix_free.hip).  Per
+// IP slot: H = du/dR by FP64 matrix instructions (inner dimension the nodes),
+// sigma and P = A' sigma in registers, f += B' P by matrix instructions (inner
+// dimension the IPs).  Every intermediate stays in the lane that needs it.
+//
+// With d.fuse (no coarse correction) and first == 0 the kernel forms the
+// direction itself, p = z + beta p with the rounding of pcg_dir_kernel: a
+// node's p is gathered by the few elements around it, so forming it in the
+// gather costs less than a kernel of its own; pcg_update stores it.  The
+// first tile then does pcg_dir_kernel's bookkeeping.
+//
+// Bound: FP64 matrix cores (HEX20 with 27 IPs: 630 v_mfma_f64_4x4x4 per group,
+// 16 cycles each: 16 us for the 64,000 elements of a 40^3 block) plus 72 B per
+// IP of geometry.  The 4x4x4 form is used because its operand and result
+// lanes agree (no exchange) and its rows need no padding to 16; measured
+// alone it reaches 68 TFLOP/s here against 43 for 16x16x4.  On the 40^3 HEX20
+// block: 33.6 us a launch, where the SpMV on the assembled matrix takes 142 us
+// (FP32 values) or 235 us (FP64); HEX20 17x19x15: 14.5 against 20.7 us; HEX8
+// 83x21x20: 11.8 against 12.5 us (FP32) and 23 (FP64), TET10 49x12x13: 9.8
+// against 23.4 and 33.7 us.
+template <int NN, int NQ>
+struct MfShape {
+    static constexpr int NS = (NN + 3) / 4, KS = (NQ + 3) / 4, HALF = KS * 3 * NS * 16;
+};
+
+template <int NN, int NQ>
+__global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ tl,
+                                                        int first)
+{
+    using S = MfShape<NN, NQ>;
+    constexpr int NS = S::NS, KS = S::KS;
+    const int2 te = tl[xcd_tile(blockIdx.x, gridDim.x)];
+    if (te.x < 0) return;
+    const SegDesc &d = D[te.x];
+    auto *ctl = glw(d.ctl);
+    if (ctl[C_DONE]) return;
+    if (ctl[C_STOP]) {
+        if (te.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
+        return;
+    }
+    __shared__ double sT[2 * S::HALF];
+    const bool fuse = d.fuse && !first;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const auto *__restrict__ p = gl(d.p);
+    const auto *__restrict__ z = gl(d.z);
+    const int64_t g0 = (int64_t)te.y * 4 * d.mfG + wave;
+    // the first group's nodes, while the tables are staged and beta is formed
+    const auto *mfconn = gl(d.mfconn);
+    int32_t nd[NS];
+    if (g0 < d.ngrp)
+#pragma unroll
+        for (int s = 0; s < NS; s++) nd[s] = mfconn[(g0 * NS + s) * 64 + lane];
+    for (int i = threadIdx.x; i < 2 * S::HALF; i += 256) sT[i] = gl(d.tab)[i];
+    double beta = 0.0;
+    const int it = ctl[C_PREV];
+    if (fuse) {
+        const int pi = (it - 1) & 1;
+        const double rzn = sum_partials<256>(d.part + (pi ? P_RZ1 : P_RZ0), d.nvblk);
+        beta = rzn / glw(d.scal)[rz_pub(1 - pi)];
+        if (te.y == 0) {
+            const double rr = sum_partials<256>(d.part + (pi ? P_RR1 : P_RR0), d.nvblk);
+            if (threadIdx.x == 0) {
+                glw(d.scal)[S_RR] = rr;
+                glw(d.scal)[S_RZ] = rzn;
+                glw(d.scal)[rz_pub(pi)] = rzn;
+                glw(d.scal)[S_BETA] = beta;
+                // stopped: the update kernel of this iteration does nothing
+                if (rr <= glw(d.scal)[S_THR] || it >= d.maxiter || !std::isfinite(rr)) ctl[C_STOP] = 1;
+                else ctl[C_ITERS] = it + 1;
+            }
+        }
+    } else if (te.y == 0 && threadIdx.x == 0) {
+        ctl[C_ITERS] = it + 1;
+    }
+    __syncthreads();
+    double pq = 0.0;
+    for (int w = 0; w < d.mfG; w++) {
+        const int64_t grp = g0 + 4 * w;
+        if (grp >= d.ngrp) break;
+        if (w > 0)
+#pragma unroll
+            for (int s = 0; s < NS; s++) nd[s] = mfconn[(grp * NS + s) * 64 + lane];
+        double u[NS][3], f[NS][3];
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                u[s][c] = p[(int64_t)nd[s] * 3 + c];
+                f[s][c] = 0.0;
+            }
+        if (fuse)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) u[s][c] = fma(beta, u[s][c], z[(int64_t)nd[s] * 3 + c]);
+        const double lam = gl(d.lm)[grp * 32 + (lane & 15)], mu = gl(d.lm)[grp * 32 + 16 + (lane & 15)];
+        const auto *geo = gl(d.geo) + grp * (KS * 9 * 64) + lane;
+#pragma unroll 1
+        for (int k = 0; k < KS; k++) {
+            double A[3][3], H[3][3];
+#pragma unroll
+            for (int r = 0; r < 9; r++) A[r / 3][r % 3] = geo[(k * 9 + r) * 64];
+            const double *t1 = sT + k * (3 * NS * 16) + (lane & 3) + 4 * (lane >> 4);
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+#pragma unroll
+                for (int c = 0; c < 3; c++) H[c][j] = 0.0;
+#pragma unroll
+                for (int s = 0; s < NS; s++) {
+                    const double a = t1[(j * NS + s) * 16];
+#pragma unroll
+                    for (int c = 0; c < 3; c++)
+                        H[c][j] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, u[s][c], H[c][j], 0, 0, 0);
+                }
+            }
+            // G = H A (du_c/dX_m), sigma = lambda tr I + mu (G + G'), P = sigma A'
+            double G[3][3], P[3][3];
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+#pragma unroll
+                for (int m = 0; m < 3; m++) G[c][m] = fma(H[c][2], A[2][m], fma(H[c][1], A[1][m], H[c][0] * A[0][m]));
+            const double lt = lam * (G[0][0] + G[1][1] + G[2][2]);
+            const double s00 = fma(2.0 * mu, G[0][0], lt), s11 = fma(2.0 * mu, G[1][1], lt),
+                         s22 = fma(2.0 * mu, G[2][2], lt);
+            const double s12 = mu * (G[1][2] + G[2][1]), s02 = mu * (G[0][2] + G[2][0]), s01 = mu * (G[0][1] + G[1][0]);
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                P[0][j] = fma(s02, A[j][2], fma(s01, A[j][1], s00 * A[j][0]));
+                P[1][j] = fma(s12, A[j][2], fma(s11, A[j][1], s01 * A[j][0]));
+                P[2][j] = fma(s22, A[j][2], fma(s12, A[j][1], s02 * A[j][0]));
+            }
+            const double *t2 = t1 + S::HALF;
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+#pragma unroll
+                for (int s = 0; s < NS; s++) {
+                    const double a = t2[(j * NS + s) * 16];
+#pragma unroll
+                    for (int c = 0; c < 3; c++)
+                        f[s][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, P[c][j], f[s][c], 0, 0, 0);
+                }
+        }
+        auto *o = glw(d.mff) + grp * (NS * 192) + lane;
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                o[(s * 3 + c) * 64] = f[s][c];
+                pq = fma(u[s][c], f[s][c], pq);
+            }
+    }
+    pq = block_sum<256>(pq);
+    if (threadIdx.x == 0) glw(d.part)[P_PQ + te.y] = pq;
+}
+
+// q of a node: its elements' products in element order, 0 at prescribed dofs
+__device__ inline void mf_node_q(const SegDesc &d, int64_t nd, double q[3])
+{
+    const auto *fp = gl(d.fptr), *src = gl(d.mfsrc);
+    const auto *f = gl(d.mff);
+    const auto *mask = gl(d.mask);
+    const int32_t k1 = fp[nd + 1];
+    double m[3], a[3] = {0.0, 0.0, 0.0};
+    for (int c = 0; c < 3; c++) m[c] = mask[nd * 3 + c];
+    // four entries' loads issued before their sums (entries past the end
+    // repeat the first one and are left out of the sum)
+    for (int32_t k = fp[nd]; k < k1; k += 4) {
+        int32_t b[4];
+        double v[4][3];
+#pragma unroll
+        for (int j = 0; j < 4; j++) b[j] = src[k + j < k1 ? k + j : k];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) v[j][c] = f[b[j] + 64 * c];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (k + j < k1)
+                for (int c = 0; c < 3; c++) a[c] += v[j][c];
+    }
+    for (int c = 0; c < 3; c++) q[c] = m[c] != 0.0 ? a[c] : 0.0;
+}
+
+// MF: members on the matrix-free operator (q summed from its element
+// products); the others read the SpMV's q.
+template <bool MF>
+__global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl,
+                                                         int first)
 {
     const int2 ve = vl[blockIdx.x];
     if (ve.x < 0) return;
     const SegDesc &d = D[ve.x];
     auto *ctl = glw(d.ctl);
     if (ctl[C_DONE]) return;
-    const int pi = (ctl[C_ITERS] - 1) & 1;
+    const bool fuse = MF && d.fuse && !first;
+    if (MF && ctl[C_STOP]) {
+        // converged before this iteration (seen by the operator's first tile)
+        if (ve.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
+        return;
+    }
+    const int iters = ctl[C_ITERS], pi = (iters - 1) & 1;
     auto *__restrict__ x = glw(d.x);
     auto *__restrict__ r = glw(d.r);
     auto *__restrict__ z = glw(d.z);
-    const auto *__restrict__ p = gl(d.p);
+    auto *__restrict__ p = glw(d.p);
     const auto *__restrict__ q = gl(d.q);
+    if (MF && ve.y == 0 && threadIdx.x == 0) ctl[C_PREV] = iters;
+    const double beta = fuse ? glw(d.scal)[S_BETA] : 0.0;
+    auto load_node = [&](int64_t n, double pv[3], double qv[3], double xv[3], double rv0[3]) {
+        for (int c = 0; c < 3; c++) {
+            pv[c] = p[n * 3 + c];
+            if (fuse) pv[c] = fma(beta, pv[c], z[n * 3 + c]);
+            xv[c] = x[n * 3 + c];
+            rv0[c] = r[n * 3 + c];
+        }
+        if (MF) mf_node_q(d, n, qv);
+        else
+            for (int c = 0; c < 3; c++) qv[c] = q[n * 3 + c];
+    };
     const int64_t stride = (int64_t)d.nvblk * WGV;
     // the first node's operands are loaded before the partial sums, so that
     // their latency overlaps the reductions
     int64_t nd = (int64_t)ve.y * WGV + threadIdx.x;
     double pv[3] = {0.0, 0.0, 0.0}, qv[3] = {0.0, 0.0, 0.0}, xv[3] = {0.0, 0.0, 0.0}, rv0[3] = {0.0, 0.0, 0.0};
-    if (nd < d.nnodes)
-        for (int c = 0; c < 3; c++) {
-            pv[c] = p[nd * 3 + c];
-            qv[c] = q[nd * 3 + c];
-            xv[c] = x[nd * 3 + c];
-            rv0[c] = r[nd * 3 + c];
-        }
-    const double pq = sum_partials<WGV>(d.part + P_PQ, d.ntiles);
+    if (nd < d.nnodes) load_node(nd, pv, qv, xv, rv0);
+    const double pq = sum_partials<WGV>(d.part + P_PQ, d.npq);
     const double rz = glw(d.scal)[rz_pub(1 - pi)];
     if (!(pq > 0.0) || !std::isfinite(pq)) {
         if (ve.y == 0 && threadIdx.x == 0) {
@@ -658,6 +876,7 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
         double rv[3], zv[3];
         for (int c = 0; c < 3; c++) {
             const int64_t i = nd * 3 + c;
+            if (fuse) p[i] = pv[c];
             x[i] = fma(a, pv[c], xv[c]);
             rv[c] = fma(-a, qv[c], rv0[c]);
             r[i] = rv[c];
@@ -669,13 +888,7 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
             rr = fma(rv[c], rv[c], rr);
         }
         nd += stride;
-        if (nd < d.nnodes)
-            for (int c = 0; c < 3; c++) {
-                pv[c] = p[nd * 3 + c];
-                qv[c] = q[nd * 3 + c];
-                xv[c] = x[nd * 3 + c];
-                rv0[c] = r[nd * 3 + c];
-            }
+        if (nd < d.nnodes) load_node(nd, pv, qv, xv, rv0);
     }
     rzn = block_sum<WGV>(rzn);
     rr = block_sum<WGV>(rr);
@@ -840,7 +1053,7 @@ __global__ void __launch_bounds__(WGV) pcg_init_kernel(const SegDesc *__restrict
     const SegDesc &d = D[ve.x];
     // iteration 0: the two-level kernels after this one write the parity
     // slot of C_ITERS - 1, i.e. slot 1, like the Jacobi partials below
-    if (ve.y == 0 && threadIdx.x == 0) glw(d.ctl)[C_ITERS] = 0;
+    if (ve.y == 0 && threadIdx.x == 0) glw(d.ctl)[C_ITERS] = glw(d.ctl)[C_PREV] = 0;
     double rz = 0.0, rr = 0.0;
     float *__restrict__ p32 = d.wp32 ? d.p32 : nullptr;
     const int64_t stride = (int64_t)d.nvblk * WGV;
@@ -919,6 +1132,7 @@ __global__ void __launch_bounds__(WGV) pcg_finalize_kernel(const SegDesc *__rest
             scal[S_GAP] = 0.0;
             scal[S_THR] = d.thr_fac * rr;
             ctl[C_ITERS] = 0;
+            ctl[C_PREV] = 0;
             ctl[C_BREAK] = 0;
             ctl[C_STOP] = 0;
             ctl[C_DONE] = rr == 0.0 ? 1 : 0;
@@ -940,6 +1154,7 @@ __global__ void __launch_bounds__(WGV) pcg_finalize_kernel(const SegDesc *__rest
         if (threadIdx.x == 0) {
             scal[S_RZ] = rz;
             scal[rz_pub(slot_pi)] = rz;
+            ctl[C_PREV] = ctl[C_ITERS];
             ctl[C_DONE] = 0;
             ctl[C_STOP] = 0;
             ctl[C_BREAK] = 0;
@@ -982,11 +1197,29 @@ Geom model_geom(const amr_model *m)
     return g;
 }
 
+// Tiles of the matrix-free operator: 4 mfG groups of 16 elements, one wave
+// per group at a time.  Up to 2,048 groups (512 workgroups, two per CU: all
+// resident at once) a wave takes one group; larger models give each wave more,
+// so that the tables are staged once per wave and the partials stay few.
+struct MfGeom {
+    int G, ntiles;
+};
+
+MfGeom mf_geom(const amr_model *m)
+{
+    MfGeom g;
+    g.G = (int)std::max<int64_t>(1, (m->mf_ngrp + 2047) / 2048);
+    g.ntiles = (int)((m->mf_ngrp + 4 * g.G - 1) / (4 * g.G));
+    return g;
+}
+
 size_t tile_lds(int R, int ndbl) { return (size_t)(((R + 1) * 4 + 15) & ~15) + (size_t)ndbl * pow2ceil(R) * 8; }
 
 // SpMV operand kinds: FP64 values; FP32 values with FP32 p and FP32
 // accumulation; FP32 values with FP64 gather and accumulation.
 enum { K_F64 = 0, K_F32, K_F32D, K_NKIND };
+// Launch groups after those: the matrix-free operator of each element shape
+enum { K_MF = K_NKIND, K_NGROUP = K_NKIND + 4 };
 
 int lanes_index(int lanes) { return lanes == 8 ? 0 : lanes == 16 ? 1 : lanes == 32 ? 2 : 3; }
 constexpr int LANES[4] = {8, 16, 32, 64};
@@ -1017,6 +1250,23 @@ void launch_pcg_spmv(int kind, int lanes, unsigned grid, int Rmax, hipStream_t s
 #undef AMR_PCG_SPMV
 }
 
+int mf_shape(const amr_model *m)
+{
+    return m->etype == AMR_HEX8 ? 0 : m->etype == AMR_TET10 ? 3 : m->nips == 27 ? 1 : 2;
+}
+
+void launch_pcg_mf(int shape, unsigned grid, hipStream_t s, const SegDesc *D, const int2 *tl, int first)
+{
+#define AMR_MF(NN, NQ) hipLaunchKernelGGL((pcg_mf_kernel<NN, NQ>), dim3(grid), dim3(256), 0, s, D, tl, first)
+    switch (shape) {
+    case 0: AMR_MF(8, 8); break;
+    case 1: AMR_MF(20, 27); break;
+    case 2: AMR_MF(20, 8); break;
+    default: AMR_MF(10, 4); break;
+    }
+#undef AMR_MF
+}
+
 void launch_residual(int lanes, unsigned grid, int Rmax, hipStream_t s, const SegDesc *D, const int2 *tl)
 {
     const size_t lds = tile_lds(Rmax, 4);
@@ -1043,6 +1293,8 @@ struct Member {
     double *x = nullptr;
     int state = 0;  // 0 free, 1 joining, 2 active
     bool mixed = false, f32x = false;
+    bool mf = false;     // iterates on the matrix-free FP64 operator
+    bool pc32 = false;   // a mixed precision was asked for: preconditioner in FP32
     double bb = 0.0, rr_ref = 0.0, rr_true_prev = INFINITY, relres = 0.0;
     int converged = 0, broke = 0, replacements = 0, iters = 0, fell_back = 0, breakdowns = 0;
     int last_rep = 0;  // iteration of the last residual replacement
@@ -1239,7 +1491,8 @@ void fill_desc(amr_pool *p, int slot)
     d.ntiles = g.ntiles;
     d.nvblk = g.nvblk;
     d.maxiter = M.o.maxiter;
-    d.f32 = M.mixed ? 1 : 0;
+    d.f32 = M.mixed || (M.mf && M.pc32) ? 1 : 0;
+    d.npq = g.ntiles;
     d.block = M.o.precond == AMR_PRECOND_BLOCK_JACOBI ? 1 : 0;
     d.wp32 = (M.mixed && M.f32x) ? 1 : 0;
     d.tl = M.o.precond == AMR_PRECOND_TWO_LEVEL ? 1 : 0;
@@ -1255,6 +1508,20 @@ void fill_desc(amr_pool *p, int slot)
         d.Kinv = m->Kinv;
         d.cvec = m->c_vec;
         d.yvec = m->y_vec;
+    }
+    if (M.mf) {
+        const MfGeom mg = mf_geom(m);
+        d.geo = m->mf_geo;
+        d.lm = m->mf_lm;
+        d.tab = m->mf_tab;
+        d.mfconn = m->mf_conn;
+        d.fptr = m->fptr;
+        d.mfsrc = m->mf_src;
+        d.mff = m->mf_f;
+        d.ngrp = m->mf_ngrp;
+        d.mfG = mg.G;
+        d.npq = mg.ntiles;
+        d.fuse = d.tl ? 0 : 1;
     }
 }
 
@@ -1308,10 +1575,15 @@ struct Group {
 void build_groups(amr_pool *p, const std::vector<int> &slots, bool residual, std::vector<std::vector<int2>> &ent,
                   std::vector<Group> &gr)
 {
-    ent.assign(K_NKIND * 4, {});
-    std::vector<int> rmax(K_NKIND * 4, 0);
+    ent.assign(K_NGROUP * 4, {});
+    std::vector<int> rmax(K_NGROUP * 4, 0);
     for (int s : slots) {
         const Member &M = p->mem[s];
+        if (M.mf && !residual) {
+            const int key = (K_MF + mf_shape(M.m)) * 4;
+            for (int t = 0; t < p->hD[s].npq; t++) ent[key].push_back(make_int2(s, t));
+            continue;
+        }
         const int kind = residual ? K_F64 : member_kind(M);
         const int key = kind * 4 + lanes_index(kind_lanes(M.m, kind));
         const SegDesc &d = p->hD[s];
@@ -1319,7 +1591,7 @@ void build_groups(amr_pool *p, const std::vector<int> &slots, bool residual, std
         rmax[key] = std::max(rmax[key], d.R);
     }
     gr.clear();
-    for (int key = 0; key < K_NKIND * 4; key++)
+    for (int key = 0; key < K_NGROUP * 4; key++)
         if (!ent[key].empty()) gr.push_back({key / 4, LANES[key % 4], rmax[key], 0, (unsigned)ent[key].size()});
 }
 
@@ -1539,7 +1811,11 @@ int amr_pool_join(amr_pool *p, amr_model *m, const double *b, double *x, const a
     M.b = b;
     M.x = x;
     M.state = M_JOIN;
-    M.mixed = o->precision == AMR_PREC_MIXED || o->precision == AMR_PREC_MIXED_F64ACC;
+    // all-elastic models iterate on the matrix-free FP64 operator in every
+    // precision: it moves fewer bytes than the FP32 matrix
+    M.pc32 = o->precision == AMR_PREC_MIXED || o->precision == AMR_PREC_MIXED_F64ACC;
+    M.mf = m->mf_ok && m->mf_plain;
+    M.mixed = M.pc32 && !M.mf;
     M.f32x = o->precision == AMR_PREC_MIXED;
     if (int rc = pool_begin_host_writes(p)) return rc;
     // the model's queued work (assembly, right-hand side) precedes its solve
@@ -1645,6 +1921,16 @@ int amr_pool_step_launch(amr_pool *p)
     if (int rc = pool_begin_host_writes(p)) return rc;
     build_groups(p, act, false, ent, gr);
     std::vector<int2> va = vec_list(p, act), aa = agg_list(p, act), ca = cw_list(p, act);
+    // members on the matrix-free operator and on an assembled matrix have
+    // update kernels of their own; vd: the members whose direction has a
+    // kernel of its own in every iteration (the others' only in the step's
+    // last one)
+    std::vector<int> sm, sa, sd;
+    for (int s : act) {
+        (p->mem[s].mf ? sm : sa).push_back(s);
+        if (!p->hD[s].fuse) sd.push_back(s);
+    }
+    std::vector<int2> vm = vec_list(p, sm), vs = vec_list(p, sa), vd = vec_list(p, sd);
     if (graph) {
         for (auto &e : ent) pad_list(e);
         int gi = 0;
@@ -1655,18 +1941,28 @@ int amr_pool_step_launch(amr_pool *p)
                 gi++;
             }
         pad_list(va);
+        pad_list(vm);
+        pad_list(vs);
+        pad_list(vd);
         pad_list(aa);
         pad_list(ca);
     }
     std::vector<int2> vj = vec_list(p, join);
     std::vector<int32_t> sj(join.begin(), join.end());
     std::vector<int2> aj = agg_list(p, join), cj = cw_list(p, join), pj = vec_list(p, tl_only(p, join));
-    size_t need = padded(vj) + padded(va) + padded(sj) + padded(aj) + padded(cj) + padded(pj) + padded(aa) +
+    size_t need = padded(vj) + padded(va) + padded(vm) + padded(vs) + padded(vd) + padded(sj) + padded(aj) + padded(cj) + padded(pj) + padded(aa) +
                   padded(ca);
     for (const auto &e : ent) need += padded(e);
     if (int rc = pool_reserve_lists(p, need)) return rc;
     Lists Ls{p};
-    const size_t o_va = Ls.push(va), o_aa = Ls.push(aa), o_ca = Ls.push(ca);
+    // a list of every member is not stored again, except for captured steps,
+    // whose offsets depend on the padded sizes alone
+    auto part = [&](const std::vector<int> &slots, const std::vector<int2> &v, size_t whole) {
+        return !graph && slots.size() == act.size() ? whole : Ls.push(v);
+    };
+    const size_t o_va = Ls.push(va);
+    const size_t o_vm = part(sm, vm, o_va), o_vs = part(sa, vs, o_va), o_vd = part(sd, vd, o_va);
+    const size_t o_aa = Ls.push(aa), o_ca = Ls.push(ca);
     {
         int gi = 0;
         for (const auto &e : ent)
@@ -1688,35 +1984,52 @@ int amr_pool_step_launch(amr_pool *p)
     auto iterations = [&]() {
         for (int j = 0; j < check; j++) {
             if (p->timing) (void)hipEventRecord(p->ev[2 * j], st);
-            for (const Group &g : gr)
-                launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, p->dD, Ls.dev_at<int2>(g.off));
+            // the step's first iteration takes p as it is (the last one of
+            // the previous step formed it)
+            const int first = j == 0 ? 1 : 0;
+            for (const Group &g : gr) {
+                if (g.kind >= K_MF)
+                    launch_pcg_mf(g.kind - K_MF, g.n, st, p->dD, Ls.dev_at<int2>(g.off), first);
+                else
+                    launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, p->dD, Ls.dev_at<int2>(g.off));
+            }
             if (p->timing) (void)hipEventRecord(p->ev[2 * j + 1], st);
-            hipLaunchKernelGGL(pcg_update_kernel, dim3((unsigned)va.size()), dim3(WGV), 0, st, p->dD,
-                               Ls.dev_at<int2>(o_va));
+            if (!vm.empty())
+                hipLaunchKernelGGL(pcg_update_kernel<true>, dim3((unsigned)vm.size()), dim3(WGV), 0, st, p->dD,
+                                   Ls.dev_at<int2>(o_vm), first);
+            if (!vs.empty())
+                hipLaunchKernelGGL(pcg_update_kernel<false>, dim3((unsigned)vs.size()), dim3(WGV), 0, st, p->dD,
+                                   Ls.dev_at<int2>(o_vs), first);
             if (!aa.empty()) {
                 hipLaunchKernelGGL(tl_restrict_kernel, dim3((unsigned)aa.size()), dim3(64), 0, st, p->dD,
                                    Ls.dev_at<int2>(o_aa), 0);
                 hipLaunchKernelGGL(tl_coarse_kernel, dim3((unsigned)ca.size()), dim3(256), 0, st, p->dD,
                                    Ls.dev_at<int2>(o_ca), 0);
             }
-            hipLaunchKernelGGL(pcg_dir_kernel, dim3((unsigned)va.size()), dim3(WGV), 0, st, p->dD,
-                               Ls.dev_at<int2>(o_va));
+            const bool last = j == check - 1;
+            if (last || !vd.empty())
+                hipLaunchKernelGGL(pcg_dir_kernel, dim3((unsigned)(last ? va.size() : vd.size())), dim3(WGV), 0, st,
+                                   p->dD, Ls.dev_at<int2>(last ? o_va : o_vd));
         }
     };
     // kernels of the step's iterations, and the host submissions that queue
     // them: one each kernel by kernel, one graph launch when captured
-    const int64_t iter_kernels = (int64_t)check * ((int64_t)gr.size() + 2 + (aa.empty() ? 0 : 2));
+    const int64_t iter_kernels =
+        (int64_t)check * ((int64_t)gr.size() + (vm.empty() ? 0 : 1) + (vs.empty() ? 0 : 1) + (aa.empty() ? 0 : 2)) +
+        (vd.empty() ? 1 : check);
     p->iter_kernels += iter_kernels;
     p->iter_submits += graph ? 1 : iter_kernels;
-    // launching each member alone would take its own SpMV, update and
+    // launching each member alone would take its own operator, update and
     // direction kernels (and restrict and coarse product, two-level) per
-    // iteration
-    for (int s : act) p->member_kernels += (int64_t)check * (p->hD[s].tl ? 5 : 3);
+    // iteration; the direction only once per step where it is fused
+    for (int s : act)
+        p->member_kernels += p->hD[s].fuse ? 2 * (int64_t)check + 1 : (int64_t)check * (p->hD[s].tl ? 5 : 3);
     if (!graph) {
         iterations();
     } else {
         std::vector<int64_t> key = {check, (int64_t)(intptr_t)p->dL, (int64_t)va.size(), (int64_t)aa.size(),
-                                    (int64_t)ca.size()};
+                                    (int64_t)ca.size(), (int64_t)vm.size(), (int64_t)vs.size(),
+                                    (int64_t)vd.size()};
         for (const Group &g : gr) key.insert(key.end(), {g.kind, g.lanes, g.Rmax, (int64_t)g.n});
         amr_pool::StepGraph *hit = nullptr;
         for (auto &g : p->graphs)
@@ -1874,15 +2187,27 @@ int step_decide(amr_pool *p, std::vector<amr_pool_result> &out)
             M.mixed = false;
             M.fell_back = 1;
             restart = true;
+        } else if (M.mf && (M.broke || M.replacements >= 2)) {
+            // the recursion on the matrix-free operator stopped above the
+            // tolerance twice, or broke down: finish on the assembled matrix,
+            // whose residual decides
+            M.mf = false;
+            M.fell_back = M.pc32 ? 1 : 0;
+            restart = true;
         } else if ((M.done && !M.broke && rr > 0.25 * M.rr_true_prev) || (M.broke && ++M.breakdowns > 3)) {
             finish(p, s, out);  // stagnation above both bounds, or repeated breakdown
             continue;
         }
         SegDesc &d = p->hD[s];
-        const int f32 = M.mixed ? 1 : 0, wp32 = (M.mixed && M.f32x) ? 1 : 0;
-        if (d.f32 != f32 || d.wp32 != wp32) {
+        const int f32 = M.mixed || (M.mf && M.pc32) ? 1 : 0, wp32 = (M.mixed && M.f32x) ? 1 : 0;
+        if (d.f32 != f32 || d.wp32 != wp32 || (d.geo && !M.mf)) {
             d.f32 = f32;
             d.wp32 = wp32;
+            if (!M.mf) {
+                d.geo = nullptr;
+                d.fuse = 0;
+                d.npq = d.ntiles;
+            }
             desc_changed = true;
         }
         M.broke = 0;

@@ -47,6 +47,12 @@ enum { AMR_PRECOND_JACOBI = 0, AMR_PRECOND_BLOCK_JACOBI = 1, AMR_PRECOND_TWO_LEV
 
 typedef struct amr_model amr_model;
 
+/* Models whose materials are all AMR_MAT_LE iterate on a matrix-free FP64
+ * operator (the elements' products from per-IP geometry, checked against the
+ * assembled FP64 matrix at the end of the solve) in every precision, which
+ * then chooses the arithmetic of the preconditioner only: FP64, or FP32 in the
+ * mixed ones.  The text of `precision` below holds for the other models, after
+ * amr_combine_KM, and for element data that mount_K's eps filter shapes. */
 typedef struct {
     int precision;      /* AMR_PREC_FP64: FP64 Jacobi-PCG.  AMR_PREC_MIXED: FP32 matrix,
                            FP32 search direction and FP32 accumulation in the SpMV,
