@@ -231,7 +231,7 @@ struct amr_model {
     bool mf_ok = false, mf_plain = false;
     int64_t mf_ngrp = 0;
     double *mf_tab = nullptr, *mf_geo = nullptr, *mf_lm = nullptr, *mf_f = nullptr;
-    int32_t *mf_conn = nullptr, *mf_src = nullptr, *mf_flag = nullptr;
+    int32_t *mf_conn = nullptr, *mf_src = nullptr, *mf_rec = nullptr, *mf_flag = nullptr;
     char *mf_block = nullptr;       // the arrays above are slices of it
     std::vector<double> mf_tab_h;   // host copy of mf_tab while it is uploaded
 };

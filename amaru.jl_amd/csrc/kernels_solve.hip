@@ -84,11 +84,38 @@ __device__ inline __attribute__((address_space(1))) T *glw(T *p)
     return (__attribute__((address_space(1))) T *)p;
 }
 
+// v of the lane that DPP control CTRL pairs with this one
+template <int CTRL>
+__device__ inline double dpp_pair(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ inline double read_lane(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Sum over the wave by one fixed tree, the same value in every lane: pairs,
+// quads, eights and rows of 16 by DPP moves (a register move each, where a
+// shuffle is an LDS round trip), then the four rows.
+__device__ inline double wave_sum(double v)
+{
+    v += dpp_pair<0xB1>(v);   // quad_perm 1,0,3,2
+    v += dpp_pair<0x4E>(v);   // quad_perm 2,3,0,1
+    v += dpp_pair<0x141>(v);  // row_half_mirror
+    v += dpp_pair<0x140>(v);  // row_mirror
+    return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
+}
+
 template <int NT>
 __device__ inline double block_sum(double v)
 {
     __shared__ double sh[NT / 64];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    v = wave_sum(v);
     __syncthreads();
     if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = v;
     __syncthreads();
@@ -110,23 +137,43 @@ __device__ inline double block_max(double v)
     return t;
 }
 
+// A thread's share of the sum of n partials (block_sum adds the shares: a
+// fixed order).
+template <int NT>
+__device__ inline double thread_partials(const double *__restrict__ P, int n)
+{
+    double v = 0.0;
+    const auto *Pg = gl(P);
+    // a thread's loads are issued before its additions, which keep the order
+    // i, i + NT, ...; addresses past the end are clamped, so that the loads
+    // need no branches
+    const int last = n - 1;
+    if (n <= 4 * NT) {
+        double a[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = (int)threadIdx.x + k * NT;
+            a[k] = Pg[i < n ? i : last];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) v = (int)threadIdx.x + k * NT < n ? v + a[k] : v;
+        return v;
+    }
+    for (int i = threadIdx.x; i < n; i += 16 * NT) {
+        double a[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) a[k] = Pg[i + k * NT < n ? i + k * NT : last];
+#pragma unroll
+        for (int k = 0; k < 16; k++) v = i + k * NT < n ? v + a[k] : v;
+    }
+    return v;
+}
+
 // Sum of n partials in a fixed order; every thread gets the result.
 template <int NT>
 __device__ inline double sum_partials(const double *__restrict__ P, int n)
 {
-    double v = 0.0;
-    // up to 16 loads of a thread issued before its additions; the additions
-    // keep the order i, i+NT, ...
-    const auto *Pg = gl(P);
-    for (int i = threadIdx.x; i < n; i += 16 * NT) {
-        double a[16];
-#pragma unroll
-        for (int k = 0; k < 16; k++) a[k] = i + k * NT < n ? Pg[i + k * NT] : 0.0;
-#pragma unroll
-        for (int k = 0; k < 16; k++)
-            if (i + k * NT < n) v += a[k];
-    }
-    return block_sum<NT>(v);
+    return block_sum<NT>(thread_partials<NT>(P, n));
 }
 
 // One model of a pool, as the kernels see it.
@@ -159,7 +206,7 @@ struct SegDesc {
     // matrix_free.hip, tiles of 4 mfG groups of 16 elements, and the map
     // node -> element products (CSR over nodes)
     const double *geo, *lm, *tab;
-    const int32_t *mfconn, *fptr, *mfsrc;
+    const int32_t *mfconn, *mfrec, *fptr, *mfsrc;
     double *mff;
     int64_t ngrp;
     int mfG;
@@ -228,6 +275,7 @@ __device__ inline void apply_prec(const SegDesc &P, int64_t node, const double r
 
 // The nine values of block k, converted to the accumulation type.
 typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
 template <typename VT, typename AT> struct BlockLoad;
 
@@ -445,6 +493,24 @@ __device__ inline double *tile_dbl(char *sm, int R, int j)
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on
 // XCD b % 8).  Entry t(b) gives each XCD one contiguous run of the work
 // list, so the slice of x a run of row tiles gathers stays in that XCD's L2.
+// Entry i of a launch's work list.  A step with one member needs none: the
+// launch passes a null list and that member's descriptor, which takes one
+// dependent load off the start of every workgroup (a pass through the kernels
+// of a small model's iteration is a chain of such loads).
+__device__ inline int2 list_entry(const int2 *__restrict__ l, int64_t i)
+{
+    return l ? l[i] : make_int2(0, (int)i);
+}
+
+// Loads written before this stay before it: the kernels of an iteration issue
+// their first loads together with the control words and only then test them,
+// and address past-the-end operands clamped instead of under a branch.  On
+// small models a wave of these kernels waits for memory three quarters of its
+// time, about 0.45 us per dependent load: with this, DPP reductions and no
+// work list, an iteration of the HEX8 20x4x4 model takes 12.0 us instead of
+// 14.6, of the HEX20 64x7x8 one 14.9 us instead of 18.0.
+#define AMR_ISSUED() asm volatile("" ::: "memory")
+
 __device__ inline int64_t xcd_tile(int64_t b, int64_t G)
 {
     const int64_t x = b & 7, i = b >> 3, q = G >> 3, rm = G & 7;
@@ -571,7 +637,7 @@ __device__ inline const float *seg_px<float>(const SegDesc &d) { return d.p32; }
 template <int L, typename VT, typename XT, typename AT>
 __global__ void __launch_bounds__(WGS) pcg_spmv_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ tl)
 {
-    const int2 te = tl[xcd_tile(blockIdx.x, gridDim.x)];
+    const int2 te = list_entry(tl, xcd_tile(blockIdx.x, gridDim.x));
     if (te.x < 0) return;  // padding of a captured step's list
     const SegDesc &d = D[te.x];
     auto *ctl = glw(d.ctl);
@@ -666,43 +732,82 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
 {
     using S = MfShape<NN, NQ>;
     constexpr int NS = S::NS, KS = S::KS;
-    const int2 te = tl[xcd_tile(blockIdx.x, gridDim.x)];
+    const int2 te = list_entry(tl, xcd_tile(blockIdx.x, gridDim.x));
     if (te.x < 0) return;
-    const SegDesc &d = D[te.x];
+    const SegDesc d = D[te.x];
     auto *ctl = glw(d.ctl);
-    if (ctl[C_DONE]) return;
-    if (ctl[C_STOP]) {
-        if (te.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
-        return;
-    }
-    __shared__ double sT[2 * S::HALF];
+    __shared__ __align__(16) double sT[2 * S::HALF];
     const bool fuse = d.fuse && !first;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const auto *__restrict__ p = gl(d.p);
-    const auto *__restrict__ z = gl(d.z);
+    // (p again, unused, where the direction is already formed)
+    const auto *__restrict__ z = fuse ? gl(d.z) : gl(d.p);
     const int64_t g0 = (int64_t)te.y * 4 * d.mfG + wave;
-    // the first group's nodes, while the tables are staged and beta is formed
     const auto *mfconn = gl(d.mfconn);
+    const int done = ctl[C_DONE], stop = ctl[C_STOP], it = ctl[C_PREV];
     int32_t nd[NS];
-    if (g0 < d.ngrp)
+    double u[NS][3], zv[NS][3], f[NS][3];
+    auto load_nodes = [&](int64_t grp) {
 #pragma unroll
-        for (int s = 0; s < NS; s++) nd[s] = mfconn[(g0 * NS + s) * 64 + lane];
-    for (int i = threadIdx.x; i < 2 * S::HALF; i += 256) sT[i] = gl(d.tab)[i];
+        for (int s = 0; s < NS; s++) nd[s] = mfconn[(grp * NS + s) * 64 + lane];
+    };
+    auto gather = [&]() {
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                u[s][c] = p[(int64_t)nd[s] * 3 + c];
+                zv[s][c] = z[(int64_t)nd[s] * 3 + c];
+            }
+    };
+    // first loads: the first group's nodes, the tables, the shares of the r.z
+    // (and, first tile, r.r) partials of both parity slots
+    load_nodes(g0 < d.ngrp ? g0 : 0);
+    constexpr int NT2 = (S::HALF + 255) / 256;  // 16-byte table loads per thread
+    f64x2 tb[NT2];
+#pragma unroll
+    for (int k = 0; k < NT2; k++) {
+        const int i = (int)threadIdx.x + k * 256;
+        tb[k] = gl((const f64x2 *)d.tab)[i < S::HALF ? i : 0];
+    }
+    double rzs[2] = {0.0, 0.0}, rrs[2] = {0.0, 0.0}, rzp[2] = {0.0, 0.0}, thr = 0.0;
+    if (fuse) {
+        rzs[0] = thread_partials<256>(d.part + P_RZ0, d.nvblk);
+        rzs[1] = thread_partials<256>(d.part + P_RZ1, d.nvblk);
+        rzp[0] = glw(d.scal)[S_RZP0];
+        rzp[1] = glw(d.scal)[S_RZP1];
+        if (te.y == 0) {
+            rrs[0] = thread_partials<256>(d.part + P_RR0, d.nvblk);
+            rrs[1] = thread_partials<256>(d.part + P_RR1, d.nvblk);
+            thr = glw(d.scal)[S_THR];
+        }
+    }
+    AMR_ISSUED();
+    if (done) return;
+    if (stop) {
+        if (te.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
+        return;
+    }
+    gather();
+#pragma unroll
+    for (int k = 0; k < NT2; k++) {
+        const int i = (int)threadIdx.x + k * 256;
+        if (i < S::HALF) ((f64x2 *)sT)[i] = tb[k];
+    }
     double beta = 0.0;
-    const int it = ctl[C_PREV];
     if (fuse) {
         const int pi = (it - 1) & 1;
-        const double rzn = sum_partials<256>(d.part + (pi ? P_RZ1 : P_RZ0), d.nvblk);
-        beta = rzn / glw(d.scal)[rz_pub(1 - pi)];
+        const double rzn = block_sum<256>(pi ? rzs[1] : rzs[0]);
+        beta = rzn / (pi ? rzp[0] : rzp[1]);
         if (te.y == 0) {
-            const double rr = sum_partials<256>(d.part + (pi ? P_RR1 : P_RR0), d.nvblk);
+            const double rr = block_sum<256>(pi ? rrs[1] : rrs[0]);
             if (threadIdx.x == 0) {
                 glw(d.scal)[S_RR] = rr;
                 glw(d.scal)[S_RZ] = rzn;
                 glw(d.scal)[rz_pub(pi)] = rzn;
                 glw(d.scal)[S_BETA] = beta;
                 // stopped: the update kernel of this iteration does nothing
-                if (rr <= glw(d.scal)[S_THR] || it >= d.maxiter || !std::isfinite(rr)) ctl[C_STOP] = 1;
+                if (rr <= thr || it >= d.maxiter || !std::isfinite(rr)) ctl[C_STOP] = 1;
                 else ctl[C_ITERS] = it + 1;
             }
         }
@@ -714,22 +819,17 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
     for (int w = 0; w < d.mfG; w++) {
         const int64_t grp = g0 + 4 * w;
         if (grp >= d.ngrp) break;
-        if (w > 0)
-#pragma unroll
-            for (int s = 0; s < NS; s++) nd[s] = mfconn[(grp * NS + s) * 64 + lane];
-        double u[NS][3], f[NS][3];
+        if (w > 0) {
+            load_nodes(grp);
+            gather();
+        }
 #pragma unroll
         for (int s = 0; s < NS; s++)
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                u[s][c] = p[(int64_t)nd[s] * 3 + c];
+                if (fuse) u[s][c] = fma(beta, u[s][c], zv[s][c]);
                 f[s][c] = 0.0;
             }
-        if (fuse)
-#pragma unroll
-            for (int s = 0; s < NS; s++)
-#pragma unroll
-                for (int c = 0; c < 3; c++) u[s][c] = fma(beta, u[s][c], z[(int64_t)nd[s] * 3 + c]);
         const double lam = gl(d.lm)[grp * 32 + (lane & 15)], mu = gl(d.lm)[grp * 32 + 16 + (lane & 15)];
         const auto *geo = gl(d.geo) + grp * (KS * 9 * 64) + lane;
 #pragma unroll 1
@@ -790,30 +890,43 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
     if (threadIdx.x == 0) glw(d.part)[P_PQ + te.y] = pq;
 }
 
-// q of a node: its elements' products in element order, 0 at prescribed dofs
-__device__ inline void mf_node_q(const SegDesc &d, int64_t nd, double q[3])
+// q of a node: its elements' products in element order, 0 at prescribed
+// dofs.  b: the node's record (matrix_free.hip), its first eight products'
+// places (-1: none); a ninth one and later ones come from the incidence list.
+__device__ inline void mf_load_q(const SegDesc &d, const int32_t b[8], double v[8][3])
 {
-    const auto *fp = gl(d.fptr), *src = gl(d.mfsrc);
     const auto *f = gl(d.mff);
-    const auto *mask = gl(d.mask);
-    const int32_t k1 = fp[nd + 1];
-    double m[3], a[3] = {0.0, 0.0, 0.0};
-    for (int c = 0; c < 3; c++) m[c] = mask[nd * 3 + c];
-    // four entries' loads issued before their sums (entries past the end
-    // repeat the first one and are left out of the sum)
-    for (int32_t k = fp[nd]; k < k1; k += 4) {
-        int32_t b[4];
-        double v[4][3];
 #pragma unroll
-        for (int j = 0; j < 4; j++) b[j] = src[k + j < k1 ? k + j : k];
+    for (int j = 0; j < 8; j++)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int c = 0; c < 3; c++) v[j][c] = f[(b[j] >= 0 ? b[j] : 0) + 64 * c];
+}
+
+__device__ inline void mf_sum_q(const SegDesc &d, int64_t nd, const int32_t b[8], double v[8][3], const double m[3],
+                                double q[3])
+{
+    double a[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-            for (int c = 0; c < 3; c++) v[j][c] = f[b[j] + 64 * c];
+    for (int j = 0; j < 8; j++)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            if (k + j < k1)
-                for (int c = 0; c < 3; c++) a[c] += v[j][c];
+        for (int c = 0; c < 3; c++) a[c] = b[j] >= 0 ? a[c] + v[j][c] : a[c];
+    if (b[7] >= 0) {
+        const auto *f = gl(d.mff);
+        const auto *fp = gl(d.fptr), *src = gl(d.mfsrc);
+        const int32_t k1 = fp[nd + 1];
+        for (int32_t k = fp[nd] + 8; k < k1; k += 4) {
+            int32_t e[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) e[j] = src[k + j < k1 ? k + j : k];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) v[j][c] = f[e[j] + 64 * c];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) a[c] = k + j < k1 ? a[c] + v[j][c] : a[c];
+        }
     }
     for (int c = 0; c < 3; c++) q[c] = m[c] != 0.0 ? a[c] : 0.0;
 }
@@ -824,44 +937,69 @@ template <bool MF>
 __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl,
                                                          int first)
 {
-    const int2 ve = vl[blockIdx.x];
+    const int2 ve = list_entry(vl, blockIdx.x);
     if (ve.x < 0) return;
-    const SegDesc &d = D[ve.x];
+    const SegDesc d = D[ve.x];
     auto *ctl = glw(d.ctl);
-    if (ctl[C_DONE]) return;
     const bool fuse = MF && d.fuse && !first;
-    if (MF && ctl[C_STOP]) {
-        // converged before this iteration (seen by the operator's first tile)
-        if (ve.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
-        return;
-    }
-    const int iters = ctl[C_ITERS], pi = (iters - 1) & 1;
+    const int done = ctl[C_DONE], stop = MF ? (int)ctl[C_STOP] : 0, iters = ctl[C_ITERS];
+    const int pi = (iters - 1) & 1;
     auto *__restrict__ x = glw(d.x);
     auto *__restrict__ r = glw(d.r);
     auto *__restrict__ z = glw(d.z);
     auto *__restrict__ p = glw(d.p);
     const auto *__restrict__ q = gl(d.q);
-    if (MF && ve.y == 0 && threadIdx.x == 0) ctl[C_PREV] = iters;
-    const double beta = fuse ? glw(d.scal)[S_BETA] : 0.0;
-    auto load_node = [&](int64_t n, double pv[3], double qv[3], double xv[3], double rv0[3]) {
-        for (int c = 0; c < 3; c++) {
-            pv[c] = p[n * 3 + c];
-            if (fuse) pv[c] = fma(beta, pv[c], z[n * 3 + c]);
-            xv[c] = x[n * 3 + c];
-            rv0[c] = r[n * 3 + c];
-        }
-        if (MF) mf_node_q(d, n, qv);
-        else
-            for (int c = 0; c < 3; c++) qv[c] = q[n * 3 + c];
+    const double beta = MF ? (double)glw(d.scal)[S_BETA] : 0.0;
+    const double rzp0 = glw(d.scal)[S_RZP0], rzp1 = glw(d.scal)[S_RZP1];
+    // z is read where the direction is formed here (else p again, unused, so
+    // that the loads need no branch)
+    const auto *zs = fuse ? gl(d.z) : gl(d.p);
+    // a node's operands; with MF also its record and mask, from which
+    // mf_load_q and mf_sum_q gather q
+    struct Node {
+        double p[3], q[3], x[3], r[3], z[3], m[3];
+        int32_t b[8];
     };
+    auto load_node = [&](int64_t n, Node &v) {
+        for (int c = 0; c < 3; c++) {
+            v.p[c] = p[n * 3 + c];
+            if (MF) v.z[c] = zs[n * 3 + c];
+            v.x[c] = x[n * 3 + c];
+            v.r[c] = r[n * 3 + c];
+            if (MF) v.m[c] = gl(d.mask)[n * 3 + c];
+            else v.q[c] = q[n * 3 + c];
+        }
+        if (MF) {
+            const auto *b = gl((const i32x4 *)d.mfrec) + 2 * n;
+            const i32x4 b0 = b[0], b1 = b[1];
+            for (int j = 0; j < 4; j++) {
+                v.b[j] = b0[j];
+                v.b[4 + j] = b1[j];
+            }
+        }
+    };
+    // the first node's operands are loaded before the control words are tested
+    // and the partials are summed, so that their latencies overlap
     const int64_t stride = (int64_t)d.nvblk * WGV;
-    // the first node's operands are loaded before the partial sums, so that
-    // their latency overlaps the reductions
     int64_t nd = (int64_t)ve.y * WGV + threadIdx.x;
-    double pv[3] = {0.0, 0.0, 0.0}, qv[3] = {0.0, 0.0, 0.0}, xv[3] = {0.0, 0.0, 0.0}, rv0[3] = {0.0, 0.0, 0.0};
-    if (nd < d.nnodes) load_node(nd, pv, qv, xv, rv0);
-    const double pq = sum_partials<WGV>(d.part + P_PQ, d.npq);
-    const double rz = glw(d.scal)[rz_pub(1 - pi)];
+    Node v = {};
+    const int64_t n0 = nd < d.nnodes ? nd : d.nnodes - 1;
+    load_node(n0, v);
+    AMR_ISSUED();
+    if (done) return;
+    if (MF && stop) {
+        // converged before this iteration (seen by the operator's first tile)
+        if (ve.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
+        return;
+    }
+    if (MF && ve.y == 0 && threadIdx.x == 0) ctl[C_PREV] = iters;
+    double fv[8][3];
+    if (MF) mf_load_q(d, v.b, fv);
+    const double pqt = thread_partials<WGV>(d.part + P_PQ, d.npq);
+    AMR_ISSUED();
+    if (MF) mf_sum_q(d, n0, v.b, fv, v.m, v.q);
+    const double pq = block_sum<WGV>(pqt);
+    const double rz = pi ? rzp0 : rzp1;
     if (!(pq > 0.0) || !std::isfinite(pq)) {
         if (ve.y == 0 && threadIdx.x == 0) {
             ctl[C_BREAK] = 1;
@@ -876,9 +1014,12 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
         double rv[3], zv[3];
         for (int c = 0; c < 3; c++) {
             const int64_t i = nd * 3 + c;
-            if (fuse) p[i] = pv[c];
-            x[i] = fma(a, pv[c], xv[c]);
-            rv[c] = fma(-a, qv[c], rv0[c]);
+            if (fuse) {
+                v.p[c] = fma(beta, v.p[c], v.z[c]);
+                p[i] = v.p[c];
+            }
+            x[i] = fma(a, v.p[c], v.x[c]);
+            rv[c] = fma(-a, v.q[c], v.r[c]);
             r[i] = rv[c];
         }
         apply_prec(d, nd, rv, zv);
@@ -888,7 +1029,13 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
             rr = fma(rv[c], rv[c], rr);
         }
         nd += stride;
-        if (nd < d.nnodes) load_node(nd, pv, qv, xv, rv0);
+        if (nd < d.nnodes) {
+            load_node(nd, v);
+            if (MF) {
+                mf_load_q(d, v.b, fv);
+                mf_sum_q(d, nd, v.b, fv, v.m, v.q);
+            }
+        }
     }
     rzn = block_sum<WGV>(rzn);
     rr = block_sum<WGV>(rr);
@@ -900,12 +1047,11 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
 
 __global__ void __launch_bounds__(WGV) pcg_dir_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl)
 {
-    const int2 ve = vl[blockIdx.x];
+    const int2 ve = list_entry(vl, blockIdx.x);
     if (ve.x < 0) return;
-    const SegDesc &d = D[ve.x];
+    const SegDesc d = D[ve.x];
     auto *ctl = glw(d.ctl);
-    if (ctl[C_DONE]) return;
-    const int it = ctl[C_ITERS], pi = (it - 1) & 1;
+    const int done = ctl[C_DONE], it = ctl[C_ITERS], pi = (it - 1) & 1;
     auto *__restrict__ p = glw(d.p);
     auto *__restrict__ p32 = d.wp32 ? glw(d.p32) : nullptr;
     const auto *__restrict__ z = gl(d.z);
@@ -917,18 +1063,32 @@ __global__ void __launch_bounds__(WGV) pcg_dir_kernel(const SegDesc *__restrict_
         pv = p[i];
         zv = d.tl ? z[i] + coarse_term(d, i / 3, (int)(i % 3)) : z[i];
     }
+    // shares of both parity slots' partials, and the published r.z
+    double rzs[2], rrs[2] = {0.0, 0.0};
+    rzs[0] = thread_partials<WGV>(d.part + P_RZ0, d.nvblk);
+    rzs[1] = thread_partials<WGV>(d.part + P_RZ1, d.nvblk);
+    if (d.tl) {
+        rzs[0] += thread_partials<WGV>(d.part + P_CY0, d.ncw);
+        rzs[1] += thread_partials<WGV>(d.part + P_CY1, d.ncw);
+    }
+    if (ve.y == 0) {
+        rrs[0] = thread_partials<WGV>(d.part + P_RR0, d.nvblk);
+        rrs[1] = thread_partials<WGV>(d.part + P_RR1, d.nvblk);
+    }
+    const double rzp0 = glw(d.scal)[S_RZP0], rzp1 = glw(d.scal)[S_RZP1], thr = glw(d.scal)[S_THR];
+    AMR_ISSUED();
+    if (done) return;
     // rz of the previous iteration was published in the other parity slot;
     // the first workgroup publishes this one's and tests convergence
-    const double rzn = sum_rz(d, pi);
-    const double rzo = glw(d.scal)[rz_pub(1 - pi)];
-    const double beta = rzn / rzo;
+    const double rzn = block_sum<WGV>(pi ? rzs[1] : rzs[0]);
+    const double beta = rzn / (pi ? rzp0 : rzp1);
     if (ve.y == 0) {
-        const double rr = sum_partials<WGV>(d.part + (pi ? P_RR1 : P_RR0), d.nvblk);
+        const double rr = block_sum<WGV>(pi ? rrs[1] : rrs[0]);
         if (threadIdx.x == 0) {
             glw(d.scal)[S_RR] = rr;
             glw(d.scal)[S_RZ] = rzn;
             glw(d.scal)[rz_pub(pi)] = rzn;
-            if (rr <= glw(d.scal)[S_THR] || it >= d.maxiter || !std::isfinite(rr)) ctl[C_STOP] = 1;
+            if (rr <= thr || it >= d.maxiter || !std::isfinite(rr)) ctl[C_STOP] = 1;
         }
     }
     while (i < n) {
@@ -951,10 +1111,10 @@ __global__ void __launch_bounds__(WGV) pcg_dir_kernel(const SegDesc *__restrict_
 __global__ void __launch_bounds__(64) tl_restrict_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ al,
                                                          int mode)
 {
-    const int2 e = al[blockIdx.x];
+    const int2 e = list_entry(al, blockIdx.x);
     if (e.x < 0) return;
-    const SegDesc &d = D[e.x];
-    if (mode == 0 && glw(d.ctl)[C_DONE]) return;
+    const SegDesc d = D[e.x];
+    const int done = mode == 0 ? (int)glw(d.ctl)[C_DONE] : 0;
     const int32_t a = e.y;
     const auto *cent = gl(d.cent), *X = gl(d.X), *rv = gl(d.r);
     const auto *aggptr = gl(d.aggptr), *aggnodes = gl(d.aggnodes);
@@ -963,8 +1123,10 @@ __global__ void __launch_bounds__(64) tl_restrict_kernel(const SegDesc *__restri
     // a lane's nodes k = k0 + lane + 64 j in order of j, eight at a time:
     // the eight nodes' loads are issued before their sums
     constexpr int NB = 8;
-    const int32_t k1 = aggptr[a + 1];
-    for (int32_t kb = aggptr[a] + threadIdx.x; kb < k1; kb += 64 * NB) {
+    const int32_t k0 = aggptr[a], k1 = aggptr[a + 1];
+    AMR_ISSUED();
+    if (done) return;
+    for (int32_t kb = k0 + threadIdx.x; kb < k1; kb += 64 * NB) {
         int64_t nd[NB];
 #pragma unroll
         for (int j = 0; j < NB; j++) nd[j] = kb + 64 * j < k1 ? aggnodes[kb + 64 * j] : -1;
@@ -998,10 +1160,10 @@ __global__ void __launch_bounds__(64) tl_restrict_kernel(const SegDesc *__restri
 __global__ void __launch_bounds__(256) tl_coarse_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ wl,
                                                         int mode)
 {
-    const int2 e = wl[blockIdx.x];
+    const int2 e = list_entry(wl, blockIdx.x);
     if (e.x < 0) return;
-    const SegDesc &d = D[e.x];
-    if (mode == 0 && glw(d.ctl)[C_DONE]) return;
+    const SegDesc d = D[e.x];
+    const int done = mode == 0 ? (int)glw(d.ctl)[C_DONE] : 0;
     const int pi = (glw(d.ctl)[C_ITERS] - 1) & 1;
     const int row = e.y * 4 + (int)(threadIdx.x / 64), lane = threadIdx.x % 64;
     double acc = 0.0;
@@ -1018,11 +1180,14 @@ __global__ void __launch_bounds__(256) tl_coarse_kernel(const SegDesc *__restric
                 kv[j] = in ? Kr[cb + 64 * j] : 0.0;
                 cv[j] = in ? cvec[cb + 64 * j] : 0.0;
             }
+            AMR_ISSUED();
+            if (done) return;  // every wave of the workgroup
 #pragma unroll
             for (int j = 0; j < NB; j++)
                 if (cb + 64 * j < d.nc) acc = fma(kv[j], cv[j], acc);
         }
     }
+    if (done) return;
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
     __shared__ double cyw[4];
     if (lane == 0) {
@@ -1517,6 +1682,7 @@ void fill_desc(amr_pool *p, int slot)
         d.mfconn = m->mf_conn;
         d.fptr = m->fptr;
         d.mfsrc = m->mf_src;
+        d.mfrec = m->mf_rec;
         d.mff = m->mf_f;
         d.ngrp = m->mf_ngrp;
         d.mfG = mg.G;
@@ -1916,11 +2082,13 @@ int amr_pool_step_launch(amr_pool *p)
     // (a) lists for the iterations (first, so that their offsets depend on
     // their own sizes only) and for the initialisation of joiners
     const bool graph = p->use_graphs && !p->timing;
+    // one member: its launches need no lists (list_entry), only their sizes
+    const bool one = !graph && act.size() == 1;
+    const SegDesc *const D = one ? p->dD + act[0] : p->dD;
     std::vector<std::vector<int2>> ent;
     std::vector<Group> gr;
     if (int rc = pool_begin_host_writes(p)) return rc;
-    build_groups(p, act, false, ent, gr);
-    std::vector<int2> va = vec_list(p, act), aa = agg_list(p, act), ca = cw_list(p, act);
+    std::vector<int2> va, aa, ca, vm, vs, vd;
     // members on the matrix-free operator and on an assembled matrix have
     // update kernels of their own; vd: the members whose direction has a
     // kernel of its own in every iteration (the others' only in the step's
@@ -1930,7 +2098,21 @@ int amr_pool_step_launch(amr_pool *p)
         (p->mem[s].mf ? sm : sa).push_back(s);
         if (!p->hD[s].fuse) sd.push_back(s);
     }
-    std::vector<int2> vm = vec_list(p, sm), vs = vec_list(p, sa), vd = vec_list(p, sd);
+    if (one) {
+        const SegDesc &d = p->hD[act[0]];
+        const Member &M = p->mem[act[0]];
+        const int kind = member_kind(M);
+        if (M.mf) gr.push_back({K_MF + mf_shape(M.m), 0, 0, 0, (unsigned)d.npq});
+        else gr.push_back({kind, kind_lanes(M.m, kind), d.R, 0, (unsigned)d.ntiles});
+    } else {
+        build_groups(p, act, false, ent, gr);
+        va = vec_list(p, act);
+        aa = agg_list(p, act);
+        ca = cw_list(p, act);
+        vm = vec_list(p, sm);
+        vs = vec_list(p, sa);
+        vd = vec_list(p, sd);
+    }
     if (graph) {
         for (auto &e : ent) pad_list(e);
         int gi = 0;
@@ -1968,6 +2150,14 @@ int amr_pool_step_launch(amr_pool *p)
         for (const auto &e : ent)
             if (!e.empty()) gr[gi++].off = Ls.push(e);
     }
+    // launch sizes, and the lists' addresses (none for one member)
+    const SegDesc &d1 = p->hD[act[0]];
+    const unsigned n_va = one ? d1.nvblk : (unsigned)va.size(), n_vm = one ? (sm.empty() ? 0 : d1.nvblk) : (unsigned)vm.size(),
+                   n_vs = one ? (sa.empty() ? 0 : d1.nvblk) : (unsigned)vs.size(),
+                   n_vd = one ? (sd.empty() ? 0 : d1.nvblk) : (unsigned)vd.size(),
+                   n_aa = one ? (d1.tl ? d1.nagg : 0) : (unsigned)aa.size(),
+                   n_ca = one ? (d1.tl ? d1.ncw : 0) : (unsigned)ca.size();
+    auto list = [&](size_t o) { return one ? (const int2 *)nullptr : Ls.dev_at<int2>(o); };
     const size_t o_vj = Ls.push(vj), o_sj = Ls.push(sj);
     const size_t o_aj = Ls.push(aj), o_cj = Ls.push(cj), o_pj = Ls.push(pj);
     if (int rc = upload(p, Ls.off, p->desc_dirty)) return rc;
@@ -1988,35 +2178,29 @@ int amr_pool_step_launch(amr_pool *p)
             // the previous step formed it)
             const int first = j == 0 ? 1 : 0;
             for (const Group &g : gr) {
-                if (g.kind >= K_MF)
-                    launch_pcg_mf(g.kind - K_MF, g.n, st, p->dD, Ls.dev_at<int2>(g.off), first);
-                else
-                    launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, p->dD, Ls.dev_at<int2>(g.off));
+                if (g.kind >= K_MF) launch_pcg_mf(g.kind - K_MF, g.n, st, D, list(g.off), first);
+                else launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, D, list(g.off));
             }
             if (p->timing) (void)hipEventRecord(p->ev[2 * j + 1], st);
-            if (!vm.empty())
-                hipLaunchKernelGGL(pcg_update_kernel<true>, dim3((unsigned)vm.size()), dim3(WGV), 0, st, p->dD,
-                                   Ls.dev_at<int2>(o_vm), first);
-            if (!vs.empty())
-                hipLaunchKernelGGL(pcg_update_kernel<false>, dim3((unsigned)vs.size()), dim3(WGV), 0, st, p->dD,
-                                   Ls.dev_at<int2>(o_vs), first);
-            if (!aa.empty()) {
-                hipLaunchKernelGGL(tl_restrict_kernel, dim3((unsigned)aa.size()), dim3(64), 0, st, p->dD,
-                                   Ls.dev_at<int2>(o_aa), 0);
-                hipLaunchKernelGGL(tl_coarse_kernel, dim3((unsigned)ca.size()), dim3(256), 0, st, p->dD,
-                                   Ls.dev_at<int2>(o_ca), 0);
+            if (n_vm)
+                hipLaunchKernelGGL(pcg_update_kernel<true>, dim3(n_vm), dim3(WGV), 0, st, D, list(o_vm), first);
+            if (n_vs)
+                hipLaunchKernelGGL(pcg_update_kernel<false>, dim3(n_vs), dim3(WGV), 0, st, D, list(o_vs), first);
+            if (n_aa) {
+                hipLaunchKernelGGL(tl_restrict_kernel, dim3(n_aa), dim3(64), 0, st, D, list(o_aa), 0);
+                hipLaunchKernelGGL(tl_coarse_kernel, dim3(n_ca), dim3(256), 0, st, D, list(o_ca), 0);
             }
             const bool last = j == check - 1;
-            if (last || !vd.empty())
-                hipLaunchKernelGGL(pcg_dir_kernel, dim3((unsigned)(last ? va.size() : vd.size())), dim3(WGV), 0, st,
-                                   p->dD, Ls.dev_at<int2>(last ? o_va : o_vd));
+            if (last || n_vd)
+                hipLaunchKernelGGL(pcg_dir_kernel, dim3(last ? n_va : n_vd), dim3(WGV), 0, st, D,
+                                   list(last ? o_va : o_vd));
         }
     };
     // kernels of the step's iterations, and the host submissions that queue
     // them: one each kernel by kernel, one graph launch when captured
     const int64_t iter_kernels =
-        (int64_t)check * ((int64_t)gr.size() + (vm.empty() ? 0 : 1) + (vs.empty() ? 0 : 1) + (aa.empty() ? 0 : 2)) +
-        (vd.empty() ? 1 : check);
+        (int64_t)check * ((int64_t)gr.size() + (n_vm ? 1 : 0) + (n_vs ? 1 : 0) + (n_aa ? 2 : 0)) +
+        (n_vd ? check : 1);
     p->iter_kernels += iter_kernels;
     p->iter_submits += graph ? 1 : iter_kernels;
     // launching each member alone would take its own operator, update and

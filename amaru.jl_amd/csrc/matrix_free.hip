@@ -106,6 +106,19 @@ __global__ void __launch_bounds__(256) mf_src_kernel(int64_t n, int NN, int NS, 
     src[p] = ((e >> 4) * NS + (a >> 2)) * 192 + (a & 3) * 16 + (e & 15);
 }
 
+// One thread per entry of the nodes' records: the places of a node's first
+// eight products (-1: fewer), 32 bytes per node read without the dependent
+// load of the list's bounds.  Nodes of structured hexahedra have at most
+// eight, most nodes of tetrahedra fewer.
+__global__ void __launch_bounds__(256) mf_rec_kernel(int64_t n, const int32_t *__restrict__ fptr,
+                                                     const int32_t *__restrict__ src, int32_t *__restrict__ rec)
+{
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= n) return;
+    const int64_t k = fptr[t >> 3] + (t & 7);
+    rec[t] = k < fptr[(t >> 3) + 1] ? src[k] : -1;
+}
+
 }  // namespace
 
 // Tables of the two products, 16 values per 4x4 block (the four blocks of an
@@ -152,7 +165,8 @@ int amr_mf_build(amr_model *m, const double *dNdR_host)
     };
     const size_t o_tab = slice(m->mf_tab_h.size() * 8), o_geo = slice((size_t)ngrp * KS * 9 * 64 * 8),
                  o_lm = slice((size_t)ngrp * 32 * 8), o_f = slice((size_t)ngrp * NS * 192 * 8),
-                 o_conn = slice((size_t)ngrp * NS * 64 * 4), o_src = slice((size_t)m->ne * NN * 4), o_flag = slice(4);
+                 o_conn = slice((size_t)ngrp * NS * 64 * 4), o_src = slice((size_t)m->ne * NN * 4), o_rec = slice((size_t)m->nnodes * 32),
+                 o_flag = slice(4);
     const int rc = amr_dalloc(m, (void **)&m->mf_block, off);
     if (rc == AMR_ERR_NOMEM) {
         // the model still fits without: it iterates on the assembled matrix
@@ -168,6 +182,7 @@ int amr_mf_build(amr_model *m, const double *dNdR_host)
     at(&m->mf_f, o_f);
     at(&m->mf_conn, o_conn);
     at(&m->mf_src, o_src);
+    at(&m->mf_rec, o_rec);
     at(&m->mf_flag, o_flag);
     hipStream_t s = m->stream;
     AMR_HIP(hipMemcpyAsync(m->mf_tab, m->mf_tab_h.data(), m->mf_tab_h.size() * sizeof(double),
@@ -179,6 +194,8 @@ int amr_mf_build(amr_model *m, const double *dNdR_host)
                        m->mats, m->dNdR, m->wip, m->mf_geo, m->mf_lm, m->mf_flag);
     hipLaunchKernelGGL(mf_conn_kernel, grid(n1), dim3(256), 0, s, n1, NN, NS, m->ne, m->conn, m->mf_conn);
     hipLaunchKernelGGL(mf_src_kernel, grid(n2), dim3(256), 0, s, n2, NN, NS, m->fsrc, m->mf_src);
+    hipLaunchKernelGGL(mf_rec_kernel, grid(m->nnodes * 8), dim3(256), 0, s, m->nnodes * 8, m->fptr, m->mf_src,
+                       m->mf_rec);
     AMR_HIP(hipGetLastError());
     return AMR_OK;
 }

@@ -484,7 +484,7 @@ def estimate_device_bytes(model):
     # matrix-free operator: geometry per IP, node ids and products per element
     # node, in groups of 16 elements
     grp = (ne + 15) // 16
-    mf = grp * (-(-nips // 4) * 4608 + -(-nn // 4) * 1792 + 256) + 4 * ne * nn + 30720 if ne else 0
+    mf = grp * (-(-nips // 4) * 4608 + -(-nn // 4) * 1792 + 256) + 4 * ne * nn + 32 * nnodes + 32768 if ne else 0
     # + the padding of the 32 vector slices (to 64 entries each)
     return int(per_node * nnodes + per_elem * ne + per_blk * (nblk + 64) + mf + 46080 * 8 + 4096 + 24 * 64 * 8 + 8 * 64 * 4)
 
