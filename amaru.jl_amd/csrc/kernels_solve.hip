@@ -203,7 +203,7 @@ struct SegDesc {
     const double *cent, *X, *Kinv;
     double *cvec, *yvec;
     // matrix-free operator (null geo: the assembled matrix): element data of
-    // matrix_free.hip, tiles of 4 mfG groups of 16 elements, and the map
+    // matrix_free.hip, tiles of mfG groups of 16 elements per wave (or team of waves), and the map
     // node -> element products (CSR over nodes)
     const double *geo, *lm, *tab;
     const int32_t *mfconn, *mfrec, *fptr, *mfsrc;
@@ -726,7 +726,7 @@ struct MfShape {
     static constexpr int NS = (NN + 3) / 4, KS = (NQ + 3) / 4, HALF = KS * 3 * NS * 16;
 };
 
-template <int NN, int NQ>
+template <int NN, int NQ, int W>
 __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ tl,
                                                         int first)
 {
@@ -738,31 +738,50 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
     auto *ctl = glw(d.ctl);
     __shared__ __align__(16) double sT[2 * S::HALF];
     const bool fuse = d.fuse && !first;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // W waves share a group, each with the IP slots sub, sub + W, ...
+    constexpr int NG = 4 / W;
+    __shared__ double sF[W > 1 ? 4 : 1][W > 1 ? NS * 192 : 1];
+    __shared__ double sU[W > 1 ? NG : 1][W > 1 ? NS * 192 : 1];
+    constexpr int NW = (NS + W - 1) / W;  // node slots gathered by a wave: sub, sub + W, ...
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = wave % W;
     const auto *__restrict__ p = gl(d.p);
     // (p again, unused, where the direction is already formed)
     const auto *__restrict__ z = fuse ? gl(d.z) : gl(d.p);
-    const int64_t g0 = (int64_t)te.y * 4 * d.mfG + wave;
+    const int64_t g0 = (int64_t)te.y * NG * d.mfG + wave / W;
     const auto *mfconn = gl(d.mfconn);
     const int done = ctl[C_DONE], stop = ctl[C_STOP], it = ctl[C_PREV];
-    int32_t nd[NS];
-    double u[NS][3], zv[NS][3], f[NS][3];
+    int32_t nd[NW];
+    double u[NS][3], pv[NW][3], zv[NW][3], f[NS][3];
     auto load_nodes = [&](int64_t grp) {
 #pragma unroll
-        for (int s = 0; s < NS; s++) nd[s] = mfconn[(grp * NS + s) * 64 + lane];
+        for (int t = 0; t < NW; t++) {
+            const int s = sub + W * t;
+            nd[t] = mfconn[(grp * NS + (s < NS ? s : 0)) * 64 + lane];
+        }
     };
     auto gather = [&]() {
 #pragma unroll
-        for (int s = 0; s < NS; s++)
+        for (int t = 0; t < NW; t++)
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                u[s][c] = p[(int64_t)nd[s] * 3 + c];
-                zv[s][c] = z[(int64_t)nd[s] * 3 + c];
+                pv[t][c] = p[(int64_t)nd[t] * 3 + c];
+                zv[t][c] = z[(int64_t)nd[t] * 3 + c];
             }
     };
-    // first loads: the first group's nodes, the tables, the shares of the r.z
+    // the geometry of an IP slot is loaded one slot ahead where waves share a
+    // group; with a group per wave the registers cost more than it hides (HEX20
+    // with 27 IPs, 40^3 block: 34.4 against 32.9 us)
+    constexpr bool AHEAD = W > 1;
+    double An[9];
+    auto load_geo = [&](int64_t grp, int k) {
+        const auto *geo = gl(d.geo) + (grp * KS + k) * 576 + lane;
+#pragma unroll
+        for (int r = 0; r < 9; r++) An[r] = geo[r * 64];
+    };
+    // first loads: the first group's nodes and geometry, the tables, the shares of the r.z
     // (and, first tile, r.r) partials of both parity slots
     load_nodes(g0 < d.ngrp ? g0 : 0);
+    if (AHEAD) load_geo(g0 < d.ngrp ? g0 : 0, sub);
     constexpr int NT2 = (S::HALF + 255) / 256;  // 16-byte table loads per thread
     f64x2 tb[NT2];
 #pragma unroll
@@ -817,26 +836,41 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
     __syncthreads();
     double pq = 0.0;
     for (int w = 0; w < d.mfG; w++) {
-        const int64_t grp = g0 + 4 * w;
-        if (grp >= d.ngrp) break;
-        if (w > 0) {
+        const int64_t grp = g0 + NG * w;
+        if (W == 1 && grp >= d.ngrp) break;  // (a shared group's waves meet at a barrier; mfG is 1 there)
+        if (W == 1 && w > 0) {
             load_nodes(grp);
+            if (AHEAD) load_geo(grp, 0);
             gather();
         }
+        // the waves of a shared group each gathered some of its nodes (the
+        // scattered loads are the L1's work, one line per lane)
+        double *su = sU[W > 1 ? wave / W : 0];
+#pragma unroll
+        for (int t = 0; t < NW; t++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const double v = fuse ? fma(beta, pv[t][c], zv[t][c]) : pv[t][c];
+                if (W == 1) u[t][c] = v;
+                else if (sub + W * t < NS) su[((sub + W * t) * 3 + c) * 64 + lane] = v;
+            }
+        if (W > 1) __syncthreads();
 #pragma unroll
         for (int s = 0; s < NS; s++)
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                if (fuse) u[s][c] = fma(beta, u[s][c], zv[s][c]);
+                if (W > 1) u[s][c] = su[(s * 3 + c) * 64 + lane];
                 f[s][c] = 0.0;
             }
-        const double lam = gl(d.lm)[grp * 32 + (lane & 15)], mu = gl(d.lm)[grp * 32 + 16 + (lane & 15)];
-        const auto *geo = gl(d.geo) + grp * (KS * 9 * 64) + lane;
+        const auto *lmp = gl(d.lm) + (grp < d.ngrp ? grp : 0) * 32 + (lane & 15);
+        const double lam = lmp[0], mu = lmp[16];
 #pragma unroll 1
-        for (int k = 0; k < KS; k++) {
+        for (int k = sub; k < KS; k += W) {
             double A[3][3], H[3][3];
+            if (!AHEAD) load_geo(grp, k);
 #pragma unroll
-            for (int r = 0; r < 9; r++) A[r / 3][r % 3] = geo[(k * 9 + r) * 64];
+            for (int r = 0; r < 9; r++) A[r / 3][r % 3] = An[r];
+            if (AHEAD && k + W < KS) load_geo(grp < d.ngrp ? grp : 0, k + W);
             const double *t1 = sT + k * (3 * NS * 16) + (lane & 3) + 4 * (lane >> 4);
 #pragma unroll
             for (int j = 0; j < 3; j++) {
@@ -882,9 +916,21 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
         for (int s = 0; s < NS; s++)
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                o[(s * 3 + c) * 64] = f[s][c];
-                pq = fma(u[s][c], f[s][c], pq);
+                if (W == 1) o[(s * 3 + c) * 64] = f[s][c];
+                else sF[wave][(s * 3 + c) * 64 + lane] = f[s][c];
+                if (W == 1 || grp < d.ngrp) pq = fma(u[s][c], f[s][c], pq);
             }
+        if (W > 1) {
+            // the group's waves add their parts, a row of 64 each in turn
+            __syncthreads();
+            if (grp < d.ngrp)
+                for (int r = sub; r < NS * 3; r += W) {
+                    double v = sF[wave - sub][r * 64 + lane];
+#pragma unroll
+                    for (int x = 1; x < W; x++) v += sF[wave - sub + x][r * 64 + lane];
+                    o[r * 64] = v;
+                }
+        }
     }
     pq = block_sum<256>(pq);
     if (threadIdx.x == 0) glw(d.part)[P_PQ + te.y] = pq;
@@ -1362,19 +1408,27 @@ Geom model_geom(const amr_model *m)
     return g;
 }
 
-// Tiles of the matrix-free operator: 4 mfG groups of 16 elements, one wave
-// per group at a time.  Up to 2,048 groups (512 workgroups, two per CU: all
-// resident at once) a wave takes one group; larger models give each wave more,
-// so that the tables are staged once per wave and the partials stay few.
+// Tiles of the matrix-free operator.  With few groups the waves of a
+// workgroup share a group where its IP slots can be divided: such a launch is
+// bound by one wave's chain of matrix instructions, not by throughput.  Four
+// waves a group for 27 IPs below 1,024 groups (a wave per SIMD; HEX20 17x19x15,
+// 303 groups: 12.3 us with one wave per group, 10.3 with four), two for the hex
+// rules with 8 IPs below 256 (HEX20 64x7x8, 224 groups: 7.2 against 6.2 us;
+// HEX8 57x15x13, 695 groups: 3% slower passes with two).  From there on a wave
+// takes a group of its own, G groups in turn only where the p.q partials would
+// not fit otherwise (two groups a wave made the 40^3 HEX20 block no faster and
+// the TET10 49x12x13 box 10% slower).
 struct MfGeom {
-    int G, ntiles;
+    int W, G, ntiles;
 };
 
 MfGeom mf_geom(const amr_model *m)
 {
     MfGeom g;
-    g.G = (int)std::max<int64_t>(1, (m->mf_ngrp + 2047) / 2048);
-    g.ntiles = (int)((m->mf_ngrp + 4 * g.G - 1) / (4 * g.G));
+    g.W = m->nips == 27 ? (m->mf_ngrp < 1024 ? 4 : 1) : m->nips == 8 ? (m->mf_ngrp < 256 ? 2 : 1) : 1;
+    const int64_t ng = 4 / g.W;
+    g.G = (int)std::max<int64_t>(1, (m->mf_ngrp + ng * MAX_GR - 1) / (ng * MAX_GR));
+    g.ntiles = (int)((m->mf_ngrp + ng * g.G - 1) / (ng * g.G));
     return g;
 }
 
@@ -1383,8 +1437,9 @@ size_t tile_lds(int R, int ndbl) { return (size_t)(((R + 1) * 4 + 15) & ~15) + (
 // SpMV operand kinds: FP64 values; FP32 values with FP32 p and FP32
 // accumulation; FP32 values with FP64 gather and accumulation.
 enum { K_F64 = 0, K_F32, K_F32D, K_NKIND };
-// Launch groups after those: the matrix-free operator of each element shape
-enum { K_MF = K_NKIND, K_NGROUP = K_NKIND + 4 };
+// Launch groups after those: the matrix-free operator of each element shape,
+// with one wave per group and with shared groups
+enum { K_MF = K_NKIND, K_NGROUP = K_NKIND + 8 };
 
 int lanes_index(int lanes) { return lanes == 8 ? 0 : lanes == 16 ? 1 : lanes == 32 ? 2 : 3; }
 constexpr int LANES[4] = {8, 16, 32, 64};
@@ -1415,19 +1470,23 @@ void launch_pcg_spmv(int kind, int lanes, unsigned grid, int Rmax, hipStream_t s
 #undef AMR_PCG_SPMV
 }
 
-int mf_shape(const amr_model *m)
+int mf_kind(const amr_model *m)
 {
-    return m->etype == AMR_HEX8 ? 0 : m->etype == AMR_TET10 ? 3 : m->nips == 27 ? 1 : 2;
+    const int shape = m->etype == AMR_HEX8 ? 0 : m->etype == AMR_TET10 ? 3 : m->nips == 27 ? 1 : 2;
+    return K_MF + 2 * shape + (mf_geom(m).W > 1 ? 1 : 0);
 }
 
-void launch_pcg_mf(int shape, unsigned grid, hipStream_t s, const SegDesc *D, const int2 *tl, int first)
+void launch_pcg_mf(int kind, unsigned grid, hipStream_t s, const SegDesc *D, const int2 *tl, int first)
 {
-#define AMR_MF(NN, NQ) hipLaunchKernelGGL((pcg_mf_kernel<NN, NQ>), dim3(grid), dim3(256), 0, s, D, tl, first)
-    switch (shape) {
-    case 0: AMR_MF(8, 8); break;
-    case 1: AMR_MF(20, 27); break;
-    case 2: AMR_MF(20, 8); break;
-    default: AMR_MF(10, 4); break;
+#define AMR_MF(NN, NQ, W) hipLaunchKernelGGL((pcg_mf_kernel<NN, NQ, W>), dim3(grid), dim3(256), 0, s, D, tl, first)
+    switch (kind - K_MF) {
+    case 0: AMR_MF(8, 8, 1); break;
+    case 1: AMR_MF(8, 8, 2); break;
+    case 2: AMR_MF(20, 27, 1); break;
+    case 3: AMR_MF(20, 27, 4); break;
+    case 4: AMR_MF(20, 8, 1); break;
+    case 5: AMR_MF(20, 8, 2); break;
+    default: AMR_MF(10, 4, 1); break;
     }
 #undef AMR_MF
 }
@@ -1746,7 +1805,7 @@ void build_groups(amr_pool *p, const std::vector<int> &slots, bool residual, std
     for (int s : slots) {
         const Member &M = p->mem[s];
         if (M.mf && !residual) {
-            const int key = (K_MF + mf_shape(M.m)) * 4;
+            const int key = mf_kind(M.m) * 4;
             for (int t = 0; t < p->hD[s].npq; t++) ent[key].push_back(make_int2(s, t));
             continue;
         }
@@ -2102,7 +2161,7 @@ int amr_pool_step_launch(amr_pool *p)
         const SegDesc &d = p->hD[act[0]];
         const Member &M = p->mem[act[0]];
         const int kind = member_kind(M);
-        if (M.mf) gr.push_back({K_MF + mf_shape(M.m), 0, 0, 0, (unsigned)d.npq});
+        if (M.mf) gr.push_back({mf_kind(M.m), 0, 0, 0, (unsigned)d.npq});
         else gr.push_back({kind, kind_lanes(M.m, kind), d.R, 0, (unsigned)d.ntiles});
     } else {
         build_groups(p, act, false, ent, gr);
@@ -2178,7 +2237,7 @@ int amr_pool_step_launch(amr_pool *p)
             // the previous step formed it)
             const int first = j == 0 ? 1 : 0;
             for (const Group &g : gr) {
-                if (g.kind >= K_MF) launch_pcg_mf(g.kind - K_MF, g.n, st, D, list(g.off), first);
+                if (g.kind >= K_MF) launch_pcg_mf(g.kind, g.n, st, D, list(g.off), first);
                 else launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, D, list(g.off));
             }
             if (p->timing) (void)hipEventRecord(p->ev[2 * j + 1], st);

@@ -55,10 +55,10 @@ def close(a, b):
     return np.linalg.norm(a - b) <= 1e-8 * np.linalg.norm(b)
 
 
-# elements: one, around a group (16) and a tile (64), and 2,049 groups (a wave
-# takes two)
+# elements: one, around a group (16) and a tile (64), and enough groups for a
+# wave each (from 256 groups; with 27 IPs from 1,024)
 SIZES = {"HEX8": [(2, 1, 1), (5, 3, 1), (4, 4, 1), (17, 1, 1), (9, 7, 1), (4, 4, 4), (13, 5, 1), (33, 32, 32)],
-         "HEX20": [(2, 1, 1), (5, 3, 1), (17, 1, 1), (13, 5, 1)],
+         "HEX20": [(2, 1, 1), (5, 3, 1), (17, 1, 1), (13, 5, 1), (26, 26, 25)],
          "TET10": [(2, 1, 1), (3, 1, 1), (11, 1, 1), (4, 3, 2)]}
 
 
