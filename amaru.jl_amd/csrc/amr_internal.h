@@ -98,6 +98,8 @@ struct AmrCoarse {
     std::vector<int32_t> cba, cbb;  // coarse blocks (a, b), ascending
     std::vector<int32_t> cbptr;     // ncb+1
     std::vector<int32_t> cbslot;    // npairs: pair slots of each coarse block, ascending row
+    std::vector<int32_t> chunk;     // 4 per chunk: first, end (places in aggnodes), aggregate, 0
+    std::vector<int32_t> aggch;     // nagg+1: chunks of each aggregate
 };
 int amr_build_coarse(int64_t nnodes, const double *X, const int32_t *rowptr, const int32_t *col, int target,
                      AmrCoarse &C);
@@ -173,6 +175,11 @@ struct amr_model {
     int32_t *c_cba = nullptr, *c_cbb = nullptr, *c_cbptr = nullptr, *c_cbslot = nullptr, *c_info = nullptr;
     double *c_cent = nullptr, *c_pair = nullptr, *Kinv = nullptr, *c_vec = nullptr, *y_vec = nullptr;
     double *c_work = nullptr;  // workspace of the coarse inversion
+    // aggregate-ordered chunks of nodes (one workgroup of the PCG vector
+    // kernels each) and their parts of Phi^T r
+    int32_t nchunk = 0;
+    int32_t *c_chunk = nullptr, *c_aggch = nullptr;
+    double *c_part = nullptr;
     // split NR finish: pinned landing area of the residual scalars and error
     // words, and the state between the two halves
     struct FinHost {

@@ -359,6 +359,23 @@ int build(amr_model *m)
     if (int rc = dev_upload(m, &m->c_agg, C.agg)) return rc;
     if (int rc = dev_upload(m, &m->c_aggptr, C.aggptr)) return rc;
     if (int rc = dev_upload(m, &m->c_aggnodes, C.aggnodes)) return rc;
+    // chunks of at most 256 k nodes (k passes of a workgroup), the smallest k
+    // that keeps the chunks' partials within their 1,024 slots
+    for (int64_t k = 1;; k++) {
+        C.chunk.clear();
+        C.aggch.assign(1, 0);
+        for (int32_t a = 0; a < C.nagg; a++) {
+            for (int64_t b = C.aggptr[a]; b < C.aggptr[a + 1]; b += 256 * k)
+                C.chunk.insert(C.chunk.end(),
+                               {(int32_t)b, (int32_t)std::min<int64_t>(C.aggptr[a + 1], b + 256 * k), a, 0});
+            C.aggch.push_back((int32_t)(C.chunk.size() / 4));
+        }
+        if (C.aggch.back() <= 1024 || 256 * k >= n) break;
+    }
+    m->nchunk = C.aggch.back();
+    if (int rc = dev_upload(m, &m->c_chunk, C.chunk)) return rc;
+    if (int rc = dev_upload(m, &m->c_aggch, C.aggch)) return rc;
+    if (int rc = dev_alloc(m, &m->c_part, (size_t)m->nchunk * 6)) return rc;
     if (int rc = dev_upload(m, &m->c_pptr, C.pptr)) return rc;
     if (int rc = dev_upload(m, &m->c_pagg, C.pagg)) return rc;
     if (int rc = dev_upload(m, &m->c_cba, C.cba)) return rc;
@@ -553,7 +570,8 @@ void amr_coarse_free(amr_model *m)
     void **ptrs[] = {(void **)&m->c_agg,  (void **)&m->c_aggptr, (void **)&m->c_aggnodes, (void **)&m->c_pptr,
                      (void **)&m->c_pagg, (void **)&m->c_cba,    (void **)&m->c_cbb,      (void **)&m->c_cbptr,
                      (void **)&m->c_cbslot, (void **)&m->c_info, (void **)&m->c_cent,     (void **)&m->c_pair,
-                     (void **)&m->Kinv,   (void **)&m->c_vec,    (void **)&m->y_vec,      (void **)&m->c_work};
+                     (void **)&m->Kinv,   (void **)&m->c_vec,    (void **)&m->y_vec,      (void **)&m->c_work,
+                     (void **)&m->c_chunk, (void **)&m->c_aggch, (void **)&m->c_part};
     for (void **p : ptrs) {
         amr_release(m, *p);
         *p = nullptr;

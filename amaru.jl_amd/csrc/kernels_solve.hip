@@ -124,6 +124,25 @@ __device__ inline double block_sum(double v)
     return t;  // same value in every thread
 }
 
+// N block sums at once; thread t < N gets sum t.
+template <int NT, int N>
+__device__ inline double block_sums(const double v[N])
+{
+    __shared__ double sh[NT / 64][N];
+    __syncthreads();
+    double w[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) w[k] = wave_sum(v[k]);
+    if (threadIdx.x % 64 == 0)
+#pragma unroll
+        for (int k = 0; k < N; k++) sh[threadIdx.x / 64][k] = w[k];
+    __syncthreads();
+    double t = 0.0;
+    if (threadIdx.x < N)
+        for (int i = 0; i < NT / 64; i++) t += sh[i][threadIdx.x];
+    return t;
+}
+
 template <int NT>
 __device__ inline double block_max(double v)
 {
@@ -176,6 +195,8 @@ __device__ inline double sum_partials(const double *__restrict__ P, int n)
     return block_sum<NT>(thread_partials<NT>(P, n));
 }
 
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+
 // One model of a pool, as the kernels see it.
 struct SegDesc {
     const int32_t *rowptr, *col;
@@ -202,6 +223,15 @@ struct SegDesc {
     const int32_t *agg, *aggptr, *aggnodes;
     const double *cent, *X, *Kinv;
     double *cvec, *yvec;
+    // the nodes in aggregate order in chunks of one workgroup each (first
+    // node, end, aggregate), the chunks of each aggregate, and the chunks'
+    // parts of c
+    const i32x4 *chunk;
+    const int32_t *aggch;
+    double *cpart;
+    int nchunk;
+    int cparts;                   // the update kernel goes by chunks and writes the parts of c
+    int nred;                     // partials of r.z and r.r from the update kernel
     // matrix-free operator (null geo: the assembled matrix): element data of
     // matrix_free.hip, tiles of mfG groups of 16 elements per wave (or team of waves), and the map
     // node -> element products (CSR over nodes)
@@ -275,7 +305,6 @@ __device__ inline void apply_prec(const SegDesc &P, int64_t node, const double r
 
 // The nine values of block k, converted to the accumulation type.
 typedef double f64x2 __attribute__((ext_vector_type(2)));
-typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
 template <typename VT, typename AT> struct BlockLoad;
 
@@ -791,13 +820,13 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
     }
     double rzs[2] = {0.0, 0.0}, rrs[2] = {0.0, 0.0}, rzp[2] = {0.0, 0.0}, thr = 0.0;
     if (fuse) {
-        rzs[0] = thread_partials<256>(d.part + P_RZ0, d.nvblk);
-        rzs[1] = thread_partials<256>(d.part + P_RZ1, d.nvblk);
+        rzs[0] = thread_partials<256>(d.part + P_RZ0, d.nred);
+        rzs[1] = thread_partials<256>(d.part + P_RZ1, d.nred);
         rzp[0] = glw(d.scal)[S_RZP0];
         rzp[1] = glw(d.scal)[S_RZP1];
         if (te.y == 0) {
-            rrs[0] = thread_partials<256>(d.part + P_RR0, d.nvblk);
-            rrs[1] = thread_partials<256>(d.part + P_RR1, d.nvblk);
+            rrs[0] = thread_partials<256>(d.part + P_RR0, d.nred);
+            rrs[1] = thread_partials<256>(d.part + P_RR1, d.nred);
             thr = glw(d.scal)[S_THR];
         }
     }
@@ -978,8 +1007,12 @@ __device__ inline void mf_sum_q(const SegDesc &d, int64_t nd, const int32_t b[8]
 }
 
 // MF: members on the matrix-free operator (q summed from its element
-// products); the others read the SpMV's q.
-template <bool MF>
+// products); the others read the SpMV's q.  TL: two-level members on an
+// assembled matrix; a workgroup takes a chunk of an aggregate's nodes and also
+// writes the chunk's part of c = Phi^T r, while r is in registers (a kernel of
+// its own for it read r and X again: 3.7 us of a 36 us iteration on the
+// 40x40x20 footing).
+template <bool MF, bool TL>
 __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl,
                                                          int first)
 {
@@ -1003,7 +1036,7 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
     // a node's operands; with MF also its record and mask, from which
     // mf_load_q and mf_sum_q gather q
     struct Node {
-        double p[3], q[3], x[3], r[3], z[3], m[3];
+        double p[3], q[3], x[3], r[3], z[3], m[3], X[3];
         int32_t b[8];
     };
     auto load_node = [&](int64_t n, Node &v) {
@@ -1014,6 +1047,7 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
             v.r[c] = r[n * 3 + c];
             if (MF) v.m[c] = gl(d.mask)[n * 3 + c];
             else v.q[c] = q[n * 3 + c];
+            if (TL) v.X[c] = gl(d.X)[n * 3 + c];
         }
         if (MF) {
             const auto *b = gl((const i32x4 *)d.mfrec) + 2 * n;
@@ -1026,11 +1060,16 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
     };
     // the first node's operands are loaded before the control words are tested
     // and the partials are summed, so that their latencies overlap
-    const int64_t stride = (int64_t)d.nvblk * WGV;
-    int64_t nd = (int64_t)ve.y * WGV + threadIdx.x;
+    // positions first + thread, + stride, ... below end: nodes, or places in
+    // the aggregate-ordered node list
+    i32x4 ch = {0, 0, 0, 0};
+    if (TL) ch = gl(d.chunk)[ve.y];
+    const int64_t stride = TL ? WGV : (int64_t)d.nvblk * WGV, end = TL ? ch.y : d.nnodes;
+    int64_t pos = (TL ? (int64_t)ch.x : (int64_t)ve.y * WGV) + threadIdx.x;
+    auto node_at = [&](int64_t k) { return TL ? (int64_t)gl(d.aggnodes)[k] : k; };
     Node v = {};
-    const int64_t n0 = nd < d.nnodes ? nd : d.nnodes - 1;
-    load_node(n0, v);
+    int64_t nd = node_at(pos < end ? pos : end - 1);
+    load_node(nd, v);
     AMR_ISSUED();
     if (done) return;
     if (MF && stop) {
@@ -1043,7 +1082,7 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
     if (MF) mf_load_q(d, v.b, fv);
     const double pqt = thread_partials<WGV>(d.part + P_PQ, d.npq);
     AMR_ISSUED();
-    if (MF) mf_sum_q(d, n0, v.b, fv, v.m, v.q);
+    if (MF) mf_sum_q(d, nd, v.b, fv, v.m, v.q);
     const double pq = block_sum<WGV>(pqt);
     const double rz = pi ? rzp0 : rzp1;
     if (!(pq > 0.0) || !std::isfinite(pq)) {
@@ -1054,9 +1093,11 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
         return;
     }
     const double a = rz / pq;
-    double rzn = 0.0, rr = 0.0;
+    double rzn = 0.0, rr = 0.0, cp[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, cen[3] = {0.0, 0.0, 0.0};
+    if (TL)
+        for (int c = 0; c < 3; c++) cen[c] = gl(d.cent)[ch.z * 3 + c];
     // one node per pass; the dot contributions in node order
-    while (nd < d.nnodes) {
+    while (pos < end) {
         double rv[3], zv[3];
         for (int c = 0; c < 3; c++) {
             const int64_t i = nd * 3 + c;
@@ -1074,8 +1115,18 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
             rzn = fma(rv[c], zv[c], rzn);
             rr = fma(rv[c], rv[c], rr);
         }
-        nd += stride;
-        if (nd < d.nnodes) {
+        if (TL) {
+            const double dx = v.X[0] - cen[0], dy = v.X[1] - cen[1], dz = v.X[2] - cen[2];
+            cp[0] += rv[0];
+            cp[1] += rv[1];
+            cp[2] += rv[2];
+            cp[3] += fma(dy, rv[2], -dz * rv[1]);
+            cp[4] += fma(dz, rv[0], -dx * rv[2]);
+            cp[5] += fma(dx, rv[1], -dy * rv[0]);
+        }
+        pos += stride;
+        if (pos < end) {
+            nd = node_at(pos);
             load_node(nd, v);
             if (MF) {
                 mf_load_q(d, v.b, fv);
@@ -1083,14 +1134,24 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
             }
         }
     }
-    rzn = block_sum<WGV>(rzn);
-    rr = block_sum<WGV>(rr);
-    if (threadIdx.x == 0) {
-        glw(d.part)[(pi ? P_RZ1 : P_RZ0) + ve.y] = rzn;
-        glw(d.part)[(pi ? P_RR1 : P_RR0) + ve.y] = rr;
-    }
+    // thread 0 writes the r.z partial, 1 the r.r one, 2..7 the part of c
+    constexpr int NSUM = TL ? 8 : 2;
+    double sums[NSUM];
+    sums[0] = rzn;
+    sums[1] = rr;
+    if (TL)
+        for (int c = 0; c < 6; c++) sums[2 + c] = cp[c];
+    const double t = block_sums<WGV, NSUM>(sums);
+    if (threadIdx.x == 0) glw(d.part)[(pi ? P_RZ1 : P_RZ0) + ve.y] = t;
+    else if (threadIdx.x == 1) glw(d.part)[(pi ? P_RR1 : P_RR0) + ve.y] = t;
+    else if (TL && threadIdx.x < 8) glw(d.cpart)[(int64_t)ve.y * 6 + threadIdx.x - 2] = t;
 }
 
+// p = z + beta p, for two-level members p = z + Phi y + beta p: a workgroup
+// takes a chunk of an aggregate's nodes, so that y and the centroid are the
+// same for all of them (per dof with the aggregate looked up: 12.9 us on the
+// 40^3 HEX20 block).
+template <bool TL>
 __global__ void __launch_bounds__(WGV) pcg_dir_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl)
 {
     const int2 ve = list_entry(vl, blockIdx.x);
@@ -1101,25 +1162,42 @@ __global__ void __launch_bounds__(WGV) pcg_dir_kernel(const SegDesc *__restrict_
     auto *__restrict__ p = glw(d.p);
     auto *__restrict__ p32 = d.wp32 ? glw(d.p32) : nullptr;
     const auto *__restrict__ z = gl(d.z);
-    const int64_t n = d.nnodes * 3, stride = (int64_t)d.nvblk * WGV;
-    // the first dof's operands (and coarse term) before the partial sums
-    int64_t i = (int64_t)ve.y * WGV + threadIdx.x;
-    double pv = 0.0, zv = 0.0;
-    if (i < n) {
-        pv = p[i];
-        zv = d.tl ? z[i] + coarse_term(d, i / 3, (int)(i % 3)) : z[i];
+    // non-TL: one dof per pass; TL: one node per pass
+    constexpr int NC = TL ? 3 : 1;
+    i32x4 ch = {0, 0, 0, 0};
+    if (TL) ch = gl(d.chunk)[ve.y];
+    const int64_t stride = TL ? WGV : (int64_t)d.nvblk * WGV, end = TL ? (int64_t)ch.y : d.nnodes * 3;
+    int64_t pos = (TL ? (int64_t)ch.x : (int64_t)ve.y * WGV) + threadIdx.x;
+    double pv[NC], zv[NC], X[NC], mk[NC];
+    int64_t i0 = 0;
+    auto load = [&](int64_t k) {
+        i0 = TL ? (int64_t)gl(d.aggnodes)[k] * 3 : k;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            pv[c] = p[i0 + c];
+            zv[c] = z[i0 + c];
+            X[c] = TL ? gl(d.X)[i0 + c] : 0.0;
+            mk[c] = TL ? gl(d.mask)[i0 + c] : 0.0;
+        }
+    };
+    // the first operands, the aggregate's correction, the shares of both
+    // parity slots' partials and the published r.z
+    load(pos < end ? pos : end - 1);
+    double y[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, cen[3] = {0.0, 0.0, 0.0};
+    if (TL) {
+        for (int c = 0; c < 6; c++) y[c] = gl(d.yvec)[(int64_t)ch.z * 6 + c];
+        for (int c = 0; c < 3; c++) cen[c] = gl(d.cent)[ch.z * 3 + c];
     }
-    // shares of both parity slots' partials, and the published r.z
     double rzs[2], rrs[2] = {0.0, 0.0};
-    rzs[0] = thread_partials<WGV>(d.part + P_RZ0, d.nvblk);
-    rzs[1] = thread_partials<WGV>(d.part + P_RZ1, d.nvblk);
-    if (d.tl) {
+    rzs[0] = thread_partials<WGV>(d.part + P_RZ0, d.nred);
+    rzs[1] = thread_partials<WGV>(d.part + P_RZ1, d.nred);
+    if (TL) {
         rzs[0] += thread_partials<WGV>(d.part + P_CY0, d.ncw);
         rzs[1] += thread_partials<WGV>(d.part + P_CY1, d.ncw);
     }
     if (ve.y == 0) {
-        rrs[0] = thread_partials<WGV>(d.part + P_RR0, d.nvblk);
-        rrs[1] = thread_partials<WGV>(d.part + P_RR1, d.nvblk);
+        rrs[0] = thread_partials<WGV>(d.part + P_RR0, d.nred);
+        rrs[1] = thread_partials<WGV>(d.part + P_RR1, d.nred);
     }
     const double rzp0 = glw(d.scal)[S_RZP0], rzp1 = glw(d.scal)[S_RZP1], thr = glw(d.scal)[S_THR];
     AMR_ISSUED();
@@ -1137,21 +1215,31 @@ __global__ void __launch_bounds__(WGV) pcg_dir_kernel(const SegDesc *__restrict_
             if (rr <= thr || it >= d.maxiter || !std::isfinite(rr)) ctl[C_STOP] = 1;
         }
     }
-    while (i < n) {
-        const double pn = fma(beta, pv, zv);
-        p[i] = pn;
-        if (p32) p32[i] = (float)pn;
-        i += stride;
-        if (i < n) {
-            pv = p[i];
-            zv = d.tl ? z[i] + coarse_term(d, i / 3, (int)(i % 3)) : z[i];
+    while (pos < end) {
+        if (TL) {
+            // Phi y at the node (coarse_term)
+            const double dx = X[0] - cen[0], dy = X[NC - 2] - cen[1], dz = X[NC - 1] - cen[2];
+            const double t[3] = {fma(-dy, y[5], fma(dz, y[4], y[0])), fma(dx, y[5], fma(-dz, y[3], y[1])),
+                                 fma(-dx, y[4], fma(dy, y[3], y[2]))};
+#pragma unroll
+            for (int c = 0; c < NC; c++) zv[c] += mk[c] != 0.0 ? t[c] : 0.0;
         }
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const double pn = fma(beta, pv[c], zv[c]);
+            p[i0 + c] = pn;
+            if (p32) p32[i0 + c] = (float)pn;
+        }
+        pos += stride;
+        if (pos < end) load(pos);
     }
 }
 
 // Two-level pieces, for the members with d.tl (mode 0: inside the iteration,
 // skipped once the member is done; mode 1: initialisation and resume)
-//   restrict: c_a = sum_{i in a} R_i^T r_i, one wave per aggregate
+//   restrict: c_a = sum_{i in a} R_i^T r_i, one wave per aggregate (inside an
+//             iteration only for the members whose update kernel does not
+//             write c's parts)
 //   coarse:   y = Kc^-1 c, one wave per coarse row, and partials of c.y
 //   prolong:  p = z + Phi y (start of a search direction)
 __global__ void __launch_bounds__(64) tl_restrict_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ al,
@@ -1212,29 +1300,52 @@ __global__ void __launch_bounds__(256) tl_coarse_kernel(const SegDesc *__restric
     const int done = mode == 0 ? (int)glw(d.ctl)[C_DONE] : 0;
     const int pi = (glw(d.ctl)[C_ITERS] - 1) & 1;
     const int row = e.y * 4 + (int)(threadIdx.x / 64), lane = threadIdx.x % 64;
-    double acc = 0.0;
-    const auto *cvec = gl(d.cvec);
-    if (row < d.nc) {
-        // columns c = lane + 64 j in order of j, sixteen loads at a time
-        const auto *Kr = gl(d.Kinv) + (int64_t)row * d.nc;
-        constexpr int NB = 16;
-        for (int cb = lane; cb < d.nc; cb += 64 * NB) {
-            double kv[NB], cv[NB];
+    // columns lane + 64 j in order of j; the first sixteen entries of the row
+    // and the workgroup's share of c are in flight together (c staged in LDS
+    // ahead of the row's loads took the kernel from 6.0 to 7.7 us on 1,020
+    // coarse dofs)
+    constexpr int NB = 16, NCV = MAX_CW * 4 / 256;
+    const auto *Kr = gl(d.Kinv) + (int64_t)(row < d.nc ? row : 0) * d.nc;
+    double kv[NB], cs[NCV];
 #pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const bool in = cb + 64 * j < d.nc;
-                kv[j] = in ? Kr[cb + 64 * j] : 0.0;
-                cv[j] = in ? cvec[cb + 64 * j] : 0.0;
-            }
-            AMR_ISSUED();
-            if (done) return;  // every wave of the workgroup
+    for (int j = 0; j < NB; j++) kv[j] = Kr[lane + 64 * j < d.nc ? lane + 64 * j : 0];
+    // c: inside an iteration from the chunks' parts where the update kernel
+    // writes them, else as tl_restrict_kernel left it
+    const bool parts = mode == 0 && d.cparts;
+    const auto *src = parts ? gl(d.cpart) : gl(d.cvec);
+    __shared__ double cvec[MAX_CW * 4];
+    if (!parts || d.nchunk == d.nagg) {
 #pragma unroll
-            for (int j = 0; j < NB; j++)
-                if (cb + 64 * j < d.nc) acc = fma(kv[j], cv[j], acc);
+        for (int t = 0; t < NCV; t++) {
+            const int k = (int)threadIdx.x + 256 * t;
+            cs[t] = src[k < d.nc ? k : 0];
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < NCV; t++) {
+            const int k = (int)threadIdx.x + 256 * t, a = k / 6, q = k - 6 * a;
+            cs[t] = 0.0;
+            if (k < d.nc)
+                for (int32_t h = gl(d.aggch)[a], h1 = gl(d.aggch)[a + 1]; h < h1; h++)
+                    cs[t] += src[(int64_t)h * 6 + q];
         }
     }
+    AMR_ISSUED();
     if (done) return;
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+#pragma unroll
+    for (int t = 0; t < NCV; t++) cvec[threadIdx.x + 256 * t] = cs[t];
+    __syncthreads();
+    double acc = 0.0;
+    if (row < d.nc)
+        for (int cb = lane; cb < d.nc; cb += 64 * NB) {
+            if (cb >= 64 * NB)
+#pragma unroll
+                for (int j = 0; j < NB; j++) kv[j] = Kr[cb + 64 * j < d.nc ? cb + 64 * j : 0];
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                acc = cb + 64 * j < d.nc ? fma(kv[j], cvec[cb + 64 * j], acc) : acc;
+        }
+    acc = wave_sum(acc);
     __shared__ double cyw[4];
     if (lane == 0) {
         if (row < d.nc) glw(d.yvec)[row] = acc;
@@ -1679,6 +1790,17 @@ int handoff(amr_model *m, hipStream_t from, hipStream_t to)
     return AMR_OK;
 }
 
+// Two-level members on an assembled matrix: the update kernel by chunks, with
+// the restriction.  On the matrix-free operator it stays in node order: summing
+// the elements' products in aggregate order lost more (TET10 49x12x13: 13.3 ->
+// 19.8 us, 40^3 HEX20: 17.6 -> 28.4 us) than the restriction's own launch (5.0
+// and 10.1 us).
+void set_cparts(SegDesc &d, bool on)
+{
+    d.cparts = on ? 1 : 0;
+    d.nred = on ? d.nchunk : d.nvblk;
+}
+
 void fill_desc(amr_pool *p, int slot)
 {
     Member &M = p->mem[slot];
@@ -1717,6 +1839,7 @@ void fill_desc(amr_pool *p, int slot)
     d.maxiter = M.o.maxiter;
     d.f32 = M.mixed || (M.mf && M.pc32) ? 1 : 0;
     d.npq = g.ntiles;
+    d.nred = g.nvblk;
     d.block = M.o.precond == AMR_PRECOND_BLOCK_JACOBI ? 1 : 0;
     d.wp32 = (M.mixed && M.f32x) ? 1 : 0;
     d.tl = M.o.precond == AMR_PRECOND_TWO_LEVEL ? 1 : 0;
@@ -1732,6 +1855,11 @@ void fill_desc(amr_pool *p, int slot)
         d.Kinv = m->Kinv;
         d.cvec = m->c_vec;
         d.yvec = m->y_vec;
+        d.chunk = (const i32x4 *)m->c_chunk;
+        d.aggch = m->c_aggch;
+        d.cpart = m->c_part;
+        d.nchunk = m->nchunk;
+        set_cparts(d, !M.mf);
     }
     if (M.mf) {
         const MfGeom mg = mf_geom(m);
@@ -1836,6 +1964,15 @@ size_t size_class(size_t n)
 void pad_list(std::vector<int2> &v)
 {
     if (!v.empty()) v.resize(size_class(v.size()), make_int2(-1, -1));
+}
+
+// the chunks of the two-level members (aggregate-ordered vector work)
+std::vector<int2> chunk_list(amr_pool *p, const std::vector<int> &slots)
+{
+    std::vector<int2> v;
+    for (int s : slots)
+        for (int j = 0; j < p->hD[s].nchunk; j++) v.push_back(make_int2(s, j));
+    return v;
 }
 
 std::vector<int2> vec_list(amr_pool *p, const std::vector<int> &slots)
@@ -2147,16 +2284,28 @@ int amr_pool_step_launch(amr_pool *p)
     std::vector<std::vector<int2>> ent;
     std::vector<Group> gr;
     if (int rc = pool_begin_host_writes(p)) return rc;
-    std::vector<int2> va, aa, ca, vm, vs, vd;
-    // members on the matrix-free operator and on an assembled matrix have
-    // update kernels of their own; vd: the members whose direction has a
-    // kernel of its own in every iteration (the others' only in the step's
-    // last one)
-    std::vector<int> sm, sa, sd;
+    // vector work: update kernels of members on the matrix-free operator, on
+    // an assembled matrix, and two-level on an assembled matrix (by chunks of
+    // their aggregates); restrictions of the matrix-free two-level members;
+    // direction kernels for the one-level members that have one in every
+    // iteration (vd), for all of them in the step's last one (vl), and for
+    // the two-level members (vt)
+    enum { V_M, V_A, V_AT, V_RS, V_D, V_L, V_T, V_CW, NV };
+    std::vector<int> sv[NV];
     for (int s : act) {
-        (p->mem[s].mf ? sm : sa).push_back(s);
-        if (!p->hD[s].fuse) sd.push_back(s);
+        const SegDesc &d = p->hD[s];
+        sv[p->mem[s].mf ? V_M : d.tl ? V_AT : V_A].push_back(s);
+        if (d.tl && p->mem[s].mf) sv[V_RS].push_back(s);
+        if (!d.tl) {
+            sv[V_L].push_back(s);
+            if (!d.fuse) sv[V_D].push_back(s);
+        } else {
+            sv[V_T].push_back(s);
+            sv[V_CW].push_back(s);
+        }
     }
+    std::vector<int2> vl[NV];
+    unsigned nv[NV];
     if (one) {
         const SegDesc &d = p->hD[act[0]];
         const Member &M = p->mem[act[0]];
@@ -2165,12 +2314,11 @@ int amr_pool_step_launch(amr_pool *p)
         else gr.push_back({kind, kind_lanes(M.m, kind), d.R, 0, (unsigned)d.ntiles});
     } else {
         build_groups(p, act, false, ent, gr);
-        va = vec_list(p, act);
-        aa = agg_list(p, act);
-        ca = cw_list(p, act);
-        vm = vec_list(p, sm);
-        vs = vec_list(p, sa);
-        vd = vec_list(p, sd);
+        for (int k = 0; k < NV; k++)
+            vl[k] = k == V_CW               ? cw_list(p, sv[k])
+                    : k == V_RS             ? agg_list(p, sv[k])
+                    : k == V_AT || k == V_T ? chunk_list(p, sv[k])
+                                            : vec_list(p, sv[k]);
     }
     if (graph) {
         for (auto &e : ent) pad_list(e);
@@ -2181,29 +2329,18 @@ int amr_pool_step_launch(amr_pool *p)
                 gr[gi].Rmax = (gr[gi].Rmax + 63) / 64 * 64;
                 gi++;
             }
-        pad_list(va);
-        pad_list(vm);
-        pad_list(vs);
-        pad_list(vd);
-        pad_list(aa);
-        pad_list(ca);
+        for (auto &v : vl) pad_list(v);
     }
     std::vector<int2> vj = vec_list(p, join);
     std::vector<int32_t> sj(join.begin(), join.end());
     std::vector<int2> aj = agg_list(p, join), cj = cw_list(p, join), pj = vec_list(p, tl_only(p, join));
-    size_t need = padded(vj) + padded(va) + padded(vm) + padded(vs) + padded(vd) + padded(sj) + padded(aj) + padded(cj) + padded(pj) + padded(aa) +
-                  padded(ca);
+    size_t need = padded(vj) + padded(sj) + padded(aj) + padded(cj) + padded(pj);
+    for (const auto &v : vl) need += padded(v);
     for (const auto &e : ent) need += padded(e);
     if (int rc = pool_reserve_lists(p, need)) return rc;
     Lists Ls{p};
-    // a list of every member is not stored again, except for captured steps,
-    // whose offsets depend on the padded sizes alone
-    auto part = [&](const std::vector<int> &slots, const std::vector<int2> &v, size_t whole) {
-        return !graph && slots.size() == act.size() ? whole : Ls.push(v);
-    };
-    const size_t o_va = Ls.push(va);
-    const size_t o_vm = part(sm, vm, o_va), o_vs = part(sa, vs, o_va), o_vd = part(sd, vd, o_va);
-    const size_t o_aa = Ls.push(aa), o_ca = Ls.push(ca);
+    size_t o_v[NV];
+    for (int k = 0; k < NV; k++) o_v[k] = Ls.push(vl[k]);
     {
         int gi = 0;
         for (const auto &e : ent)
@@ -2211,11 +2348,13 @@ int amr_pool_step_launch(amr_pool *p)
     }
     // launch sizes, and the lists' addresses (none for one member)
     const SegDesc &d1 = p->hD[act[0]];
-    const unsigned n_va = one ? d1.nvblk : (unsigned)va.size(), n_vm = one ? (sm.empty() ? 0 : d1.nvblk) : (unsigned)vm.size(),
-                   n_vs = one ? (sa.empty() ? 0 : d1.nvblk) : (unsigned)vs.size(),
-                   n_vd = one ? (sd.empty() ? 0 : d1.nvblk) : (unsigned)vd.size(),
-                   n_aa = one ? (d1.tl ? d1.nagg : 0) : (unsigned)aa.size(),
-                   n_ca = one ? (d1.tl ? d1.ncw : 0) : (unsigned)ca.size();
+    for (int k = 0; k < NV; k++)
+        nv[k] = !one            ? (unsigned)vl[k].size()
+                : sv[k].empty() ? 0
+                : k == V_CW     ? (unsigned)d1.ncw
+                : k == V_RS     ? (unsigned)d1.nagg
+                : k == V_AT || k == V_T ? (unsigned)d1.nchunk
+                                        : (unsigned)d1.nvblk;
     auto list = [&](size_t o) { return one ? (const int2 *)nullptr : Ls.dev_at<int2>(o); };
     const size_t o_vj = Ls.push(vj), o_sj = Ls.push(sj);
     const size_t o_aj = Ls.push(aj), o_cj = Ls.push(cj), o_pj = Ls.push(pj);
@@ -2241,38 +2380,37 @@ int amr_pool_step_launch(amr_pool *p)
                 else launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, D, list(g.off));
             }
             if (p->timing) (void)hipEventRecord(p->ev[2 * j + 1], st);
-            if (n_vm)
-                hipLaunchKernelGGL(pcg_update_kernel<true>, dim3(n_vm), dim3(WGV), 0, st, D, list(o_vm), first);
-            if (n_vs)
-                hipLaunchKernelGGL(pcg_update_kernel<false>, dim3(n_vs), dim3(WGV), 0, st, D, list(o_vs), first);
-            if (n_aa) {
-                hipLaunchKernelGGL(tl_restrict_kernel, dim3(n_aa), dim3(64), 0, st, D, list(o_aa), 0);
-                hipLaunchKernelGGL(tl_coarse_kernel, dim3(n_ca), dim3(256), 0, st, D, list(o_ca), 0);
-            }
-            const bool last = j == check - 1;
-            if (last || n_vd)
-                hipLaunchKernelGGL(pcg_dir_kernel, dim3(last ? n_va : n_vd), dim3(WGV), 0, st, D,
-                                   list(last ? o_va : o_vd));
+            auto launch = [&](int k, auto kernel, int threads, auto... args) {
+                if (nv[k])
+                    hipLaunchKernelGGL(kernel, dim3(nv[k]), dim3(threads), 0, st, D, list(o_v[k]), args...);
+            };
+            launch(V_M, pcg_update_kernel<true, false>, WGV, first);
+            launch(V_A, pcg_update_kernel<false, false>, WGV, first);
+            launch(V_AT, pcg_update_kernel<false, true>, WGV, first);
+            launch(V_RS, tl_restrict_kernel, 64, 0);
+            launch(V_CW, tl_coarse_kernel, 256, 0);
+            launch(j == check - 1 ? V_L : V_D, pcg_dir_kernel<false>, WGV);
+            launch(V_T, pcg_dir_kernel<true>, WGV);
         }
     };
     // kernels of the step's iterations, and the host submissions that queue
     // them: one each kernel by kernel, one graph launch when captured
+    auto has = [&](int k) { return (int64_t)(nv[k] ? 1 : 0); };
     const int64_t iter_kernels =
-        (int64_t)check * ((int64_t)gr.size() + (n_vm ? 1 : 0) + (n_vs ? 1 : 0) + (n_aa ? 2 : 0)) +
-        (n_vd ? check : 1);
+        (int64_t)check * ((int64_t)gr.size() + has(V_M) + has(V_A) + has(V_AT) + has(V_RS) + has(V_CW) + has(V_T)) +
+        (check - 1) * has(V_D) + has(V_L);
     p->iter_kernels += iter_kernels;
     p->iter_submits += graph ? 1 : iter_kernels;
     // launching each member alone would take its own operator, update and
     // direction kernels (and restrict and coarse product, two-level) per
     // iteration; the direction only once per step where it is fused
     for (int s : act)
-        p->member_kernels += p->hD[s].fuse ? 2 * (int64_t)check + 1 : (int64_t)check * (p->hD[s].tl ? 5 : 3);
+        p->member_kernels += p->hD[s].fuse ? 2 * (int64_t)check + 1 : (int64_t)check * (p->hD[s].tl ? (p->hD[s].cparts ? 4 : 5) : 3);
     if (!graph) {
         iterations();
     } else {
-        std::vector<int64_t> key = {check, (int64_t)(intptr_t)p->dL, (int64_t)va.size(), (int64_t)aa.size(),
-                                    (int64_t)ca.size(), (int64_t)vm.size(), (int64_t)vs.size(),
-                                    (int64_t)vd.size()};
+        std::vector<int64_t> key = {check, (int64_t)(intptr_t)p->dL};
+        for (const auto &v : vl) key.push_back((int64_t)v.size());
         for (const Group &g : gr) key.insert(key.end(), {g.kind, g.lanes, g.Rmax, (int64_t)g.n});
         amr_pool::StepGraph *hit = nullptr;
         for (auto &g : p->graphs)
@@ -2450,6 +2588,7 @@ int step_decide(amr_pool *p, std::vector<amr_pool_result> &out)
                 d.geo = nullptr;
                 d.fuse = 0;
                 d.npq = d.ntiles;
+                if (d.tl) set_cparts(d, true);
             }
             desc_changed = true;
         }

@@ -1,0 +1,43 @@
+"""GPU: the two-level iteration's chunks (update with restriction, coarse
+product, direction by chunks of an aggregate's nodes) at their edges: one
+aggregate, and aggregates below, at and above one workgroup's 256 nodes.
+
+The solution does not depend on the preconditioner: bar 1e-8 against the
+oracle's direct solve (solves to a relative residual of 1e-12).  The
+Drucker-Prager material keeps the assembled matrix, where the update kernel
+works by chunks; the elastic one takes the matrix-free operator, where it
+does not.
+"""
+import numpy as np
+import pytest
+
+from oracle import HEX8 as O8, fem
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("plastic", [True, False])
+@pytest.mark.parametrize("target", [40, 255, 256, 300, 700, 100000])
+@pytest.mark.parametrize("precision", ["fp64", "mixed64acc"])
+def test_chunks_match_direct(amaru, plastic, target, precision):
+    am = amaru
+    mesh = am.Mesh(am.Block([[0, 0, 0], [2.0, 1.0, 1.0]], nx=13, ny=9, nz=8, cellshape="HEX8"))
+    prm = (50e6, 0.3, 0.23094, 24000.0, 0.0)
+    mat = (am.DruckerPrager(E=prm[0], nu=prm[1], alpha=prm[2], kappa=prm[3], H=prm[4]) if plastic
+           else am.LinearElastic(E=prm[0], nu=prm[1]))
+    model = am.FEModel(mesh, [("all", am.MechSolid, mat)])
+    bcs = {"x==0": dict(ux=0, uy=0, uz=0), "x==2": dict(tz=-1e3)}
+    model.configure_dofs([(f, am.SurfaceBC(**c)) for f, c in bcs.items()])
+    om = fem.Model(mesh.coords, mesh.conn, O8, [("LinearElastic", prm[:2])])
+    om.configure_dofs([(f, fem.SurfaceBC(**c)) for f, c in bcs.items()])
+    Uo, Fo = model.bc_vals([(f, am.SurfaceBC(**c)) for f, c in bcs.items()])
+    U, F = Uo.copy(), Fo.copy()
+    fem.solve_system(om.mount_K().tocsr(), Uo, Fo, om.nu)
+    dev = am.DeviceModel(model)
+    dev.set_coarse(target)
+    dev.assemble()
+    r = dev.solve_system(U, F, rtol=1e-12, precision=precision, precond="two_level")
+    assert r["converged"]
+    assert np.linalg.norm(U - Uo) <= 1e-8 * np.linalg.norm(Uo)
+    assert np.linalg.norm(F - Fo) <= 1e-8 * np.linalg.norm(Fo)
+    dev.close()
