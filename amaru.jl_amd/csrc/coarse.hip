@@ -27,6 +27,7 @@
 #include <cstring>
 
 #include "amr_internal.h"
+#include "wave_ops.h"
 
 namespace {
 
@@ -112,8 +113,7 @@ __global__ void __launch_bounds__(256) galerkin_pairs_kernel(const CoarseJob *__
                                       fma(Kb[r * 3 + 1], R[1][c], fma(Kb[r * 3], R[0][c], W[r][c])));
             }
             for (int r = 0; r < 3; r++)
-                for (int c = 0; c < 6; c++)
-                    for (int off = 32; off > 0; off >>= 1) W[r][c] += __shfl_xor(W[r][c], off, 64);
+                for (int c = 0; c < 6; c++) W[r][c] = wave_sum(W[r][c]);
             if (lane == 0) {
                 const int32_t a = agg[i];
                 double d[3], mk[3], R[3][6];
@@ -153,8 +153,8 @@ __global__ void __launch_bounds__(256) galerkin_blocks_kernel(const CoarseJob *_
     }
     double out = 0.0;
     for (int c = 0; c < 36; c++) {
-        for (int off = 32; off > 0; off >>= 1) acc[c] += __shfl_xor(acc[c], off, 64);
-        if (lane == c) out = acc[c];
+        const double t = wave_sum(acc[c]);
+        if (lane == c) out = t;
     }
     if (lane < 36)
         cgw(q.Kc)[(int64_t)(6 * cg(q.cba)[cb] + lane / 6) * q.nc + 6 * cg(q.cbb)[cb] + lane % 6] = out;
@@ -209,44 +209,115 @@ __global__ void __launch_bounds__(256) symmetrize_kernel(const CoarseJob *__rest
 //   R    = P A_Kj for j outside K; C = A_iK     (gj_panel, old column panel)
 //   A_ij -= C_i R_j,  A_Kj = R_j,  A_iK = -C_i P,  A_KK = P      (gj_update)
 // A launch does step k for every listed model with more than k block rows.
+//
+// The 64x64x64 products run on the FP64 matrix cores (v_mfma_f64_16x16x4: a wave
+// takes 16 columns of the tile, four row tiles, 16 steps over the inner
+// dimension; operand lanes m or n + 16 k, result rows l / 16 + 4 r), with the
+// operands in LDS at strides that spread a wave's lanes over the banks.  Bound
+// by latency: one step's launches are a chain.  For 1,536 coarse dofs (24
+// steps) pivot + panel + update took 72 + 47 + 52 us a step with scalar
+// products and a pivot elimination of 64 barrier steps, now 26 + 17 + 29.
 constexpr int GJB = 64;
+constexpr int SA = 68, SB = 80;  // LDS row strides of the left and right operands
 
-// entry (job, -): the pivot block of step k
-__global__ void __launch_bounds__(1024) gj_pivot_kernel(const CoarseJob *__restrict__ J, const int2 *__restrict__ wl,
-                                                        int32_t k)
+typedef double f64x4c __attribute__((ext_vector_type(4)));
+
+// acc[mt] += (rows 16 mt .. of A) (columns 16 nt .. of B) over KS steps of 4
+template <int MT, int KS>
+__device__ inline void mm_tiles(const double *A, const double *B, int lane, f64x4c acc[MT])
+{
+    const int m = lane & 15, kk = lane >> 4;
+#pragma unroll 4
+    for (int s = 0; s < KS; s++) {
+        const double b = B[(4 * s + kk) * SB + m];
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+            acc[mt] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[(16 * mt + m) * SA + 4 * s + kk], b, acc[mt], 0, 0, 0);
+    }
+}
+
+// In-place inverse of a 16x16 block held by one wave: lane l has row l / 4,
+// columns 4 (l % 4) .. + 3.  Gauss-Jordan without pivoting; the pivot row
+// comes by shuffles, the pivot column inside each quad.
+__device__ inline bool invert16(double v[4], int lane)
+{
+    bool good = true;
+    const int i = lane >> 2, q = lane & 3;
+#pragma unroll
+    for (int p = 0; p < 16; p++) {
+        const double piv = read_lane(v[p & 3], 4 * p + (p >> 2));
+        const bool ok = piv > 0.0 && std::isfinite(piv);
+        good = good && ok;
+        const double ip = ok ? 1.0 / piv : 0.0;
+        double rj[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) rj[c] = __shfl(v[c], 4 * p + q, 64) * ip;
+        constexpr int Q[4] = {0x00, 0x55, 0xAA, 0xFF};
+        const double ci = (p >> 2) == 0   ? dpp_pair<Q[0]>(v[p & 3])
+                          : (p >> 2) == 1 ? dpp_pair<Q[1]>(v[p & 3])
+                          : (p >> 2) == 2 ? dpp_pair<Q[2]>(v[p & 3])
+                                          : dpp_pair<Q[3]>(v[p & 3]);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const bool jp = 4 * q + c == p;
+            const double row = jp ? ip : rj[c];
+            const double rest = jp ? -(ci * ip) : v[c] - ci * rj[c];
+            v[c] = i == p ? row : rest;
+        }
+    }
+    return good;
+}
+
+// entry (job, -): the pivot block of step k, inverted in LDS by four block
+// steps of 16: the diagonal block by one wave in registers, the rest as
+// products.  A short last block is padded with the identity.
+__global__ void __launch_bounds__(256) gj_pivot_kernel(const CoarseJob *__restrict__ J, const int2 *__restrict__ wl,
+                                                       int32_t k)
 {
     const CoarseJob &q = J[wl[blockIdx.x].x];
     const int32_t nc = q.nc, k0 = k * GJB, b = nc - k0 < GJB ? nc - k0 : GJB;
     const auto *__restrict__ A = cg(q.Kc);
     auto *__restrict__ P = cgw(q.P);
-    // the pivot block in LDS; thread (i, j0) updates entries (i, j0..j0+3):
-    // each step reads the pivot row and column, then (after a barrier)
-    // writes the new values
-    __shared__ double M[GJB][GJB + 1];
-    const int i = threadIdx.x >> 4, j0 = (threadIdx.x & 15) * 4;
-    for (int c = 0; c < 4; c++) M[i][j0 + c] = (i < b && j0 + c < b) ? A[(int64_t)(k0 + i) * nc + k0 + j0 + c] : 0.0;
+    // M is read as the left operand (stride SA); the pivot rows, P16 on the
+    // left and the new rows on the right have copies of their own
+    __shared__ double M[GJB * SA], sP[16 * SA], sR[16 * SB];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, kk = lane >> 4;
+    for (int r = w; r < GJB; r += 4)
+        M[r * SA + lane] = (r < b && lane < b) ? A[(int64_t)(k0 + r) * nc + k0 + lane] : (r == lane ? 1.0 : 0.0);
     __syncthreads();
-    for (int p = 0; p < b; p++) {
-        const double piv = M[p][p];
-        const bool ok = piv > 0.0 && std::isfinite(piv);
-        if (!ok && threadIdx.x == 0) cgw(q.info)[0] = 1;
-        const double ip = ok ? 1.0 / piv : 0.0;
-        const double ci = M[i][p];
-        double nv[4];
-        for (int c = 0; c < 4; c++) {
-            const int j = j0 + c;
-            const double rj = M[p][j], v = M[i][j];
-            if (i == p && j == p) nv[c] = ip;
-            else if (i == p) nv[c] = rj * ip;
-            else if (j == p) nv[c] = -(ci * ip);
-            else nv[c] = v - ci * (rj * ip);
+    for (int kb = 0; kb < 4; kb++) {
+        const int o = 16 * kb;
+        if (w == 0) {
+            double v[4];
+            for (int c = 0; c < 4; c++) v[c] = M[(o + (lane >> 2)) * SA + o + 4 * (lane & 3) + c];
+            if (!invert16(v, lane) && lane == 0) cgw(q.info)[0] = 1;
+            for (int c = 0; c < 4; c++) sP[(lane >> 2) * SA + 4 * (lane & 3) + c] = v[c];
         }
+        // the pivot rows as a right operand
+        for (int r = w; r < 16; r += 4) sR[r * SB + lane] = M[(o + r) * SA + lane];
         __syncthreads();
-        for (int c = 0; c < 4; c++) M[i][j0 + c] = nv[c];
+        // wave w: columns 16 w ..  New rows R = P16 M_k (P16 itself at kb)
+        f64x4c R[1] = {f64x4c{0.0, 0.0, 0.0, 0.0}};
+        mm_tiles<1, 4>(sP, sR + 16 * w, lane, R);
+        if (w == kb)
+            for (int r = 0; r < 4; r++) R[0][r] = sP[(kk + 4 * r) * SA + m];
+        __syncthreads();
+        for (int r = 0; r < 4; r++) sR[(kk + 4 * r) * SB + 16 * w + m] = R[0][r];
+        __syncthreads();
+        // C_i R for every row tile, from the old column panel
+        f64x4c acc[4];
+        for (int mt = 0; mt < 4; mt++) acc[mt] = f64x4c{0.0, 0.0, 0.0, 0.0};
+        mm_tiles<4, 4>(M + o, sR + 16 * w, lane, acc);
+        __syncthreads();
+        for (int mt = 0; mt < 4; mt++)
+            for (int r = 0; r < 4; r++) {
+                double &x = M[(16 * mt + kk + 4 * r) * SA + 16 * w + m];
+                x = mt == kb ? R[0][r] : w == kb ? -acc[mt][r] : x - acc[mt][r];
+            }
         __syncthreads();
     }
-    for (int c = 0; c < 4; c++)
-        if (i < b && j0 + c < b) P[i * GJB + j0 + c] = M[i][j0 + c];
+    for (int r = w; r < b; r += 4)
+        if (lane < b) P[r * GJB + lane] = M[r * SA + lane];
 }
 
 // entry (job, t), one per 64-column tile t: R[:, tile] = P A_K,tile (t != k),
@@ -259,29 +330,28 @@ __global__ void __launch_bounds__(256) gj_panel_kernel(const CoarseJob *__restri
     const int32_t nc = q.nc, t = e.y, k0 = k * GJB, c0 = t * GJB, b = nc - k0 < GJB ? nc - k0 : GJB;
     const auto *__restrict__ A = cg(q.Kc), *__restrict__ P = cg(q.P);
     auto *__restrict__ R = cgw(q.R), *__restrict__ C = cgw(q.C);
-    __shared__ double Ps[GJB][GJB + 1];
-    __shared__ double As[GJB][GJB + 1];
-    const int w = std::min(GJB, nc - c0);  // columns (and rows) of this tile
-    const int r = threadIdx.x >> 2, q0 = (threadIdx.x & 3) * 16;  // 64 rows x 4 quarters
-    if (r < w)
-        for (int c = q0; c < q0 + 16 && c < b; c++) C[(int64_t)(c0 + r) * GJB + c] = A[(int64_t)(c0 + r) * nc + k0 + c];
+    __shared__ double Ps[GJB * SA], As[GJB * SB];
+    const int n = std::min(GJB, nc - c0);  // columns (and rows) of this tile
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, kk = lane >> 4;
+#pragma unroll 4
+    for (int r = w; r < GJB; r += 4) {
+        if (r < n && lane < b) C[(int64_t)(c0 + r) * GJB + lane] = A[(int64_t)(c0 + r) * nc + k0 + lane];
+        Ps[r * SA + lane] = r < b && lane < b ? P[r * GJB + lane] : 0.0;
+        As[r * SB + lane] = r < b && lane < n ? A[(int64_t)(k0 + r) * nc + c0 + lane] : 0.0;
+    }
     if (t == k) return;
-    if (r < b)
-        for (int c = q0; c < q0 + 16; c++) {
-            if (c < b) Ps[r][c] = P[r * GJB + c];
-            if (c < w) As[r][c] = A[(int64_t)(k0 + r) * nc + c0 + c];
-        }
     __syncthreads();
-    if (r < b)
-        for (int c = q0; c < q0 + 16 && c < w; c++) {
-            double acc = 0.0;
-            for (int l = 0; l < b; l++) acc = fma(Ps[r][l], As[l][c], acc);
-            R[(int64_t)r * nc + c0 + c] = acc;
+    f64x4c acc[4];
+    for (int mt = 0; mt < 4; mt++) acc[mt] = f64x4c{0.0, 0.0, 0.0, 0.0};
+    mm_tiles<4, 16>(Ps, As + 16 * w, lane, acc);
+    for (int mt = 0; mt < 4; mt++)
+        for (int r = 0; r < 4; r++) {
+            const int row = 16 * mt + kk + 4 * r, col = 16 * w + m;
+            if (row < b && col < n) R[(int64_t)row * nc + c0 + col] = acc[mt][r];
         }
 }
 
-// entry (job, ti * nt + tj), one per 64x64 tile (ti, tj) of A, 4x4 entries
-// per thread
+// entry (job, ti * nt + tj), one per 64x64 tile (ti, tj) of A
 __global__ void __launch_bounds__(256) gj_update_kernel(const CoarseJob *__restrict__ J, const int2 *__restrict__ wl,
                                                         int32_t k)
 {
@@ -291,41 +361,37 @@ __global__ void __launch_bounds__(256) gj_update_kernel(const CoarseJob *__restr
     const int32_t b = nc - k0 < GJB ? nc - k0 : GJB;
     auto *__restrict__ A = cgw(q.Kc);
     const auto *__restrict__ P = cg(q.P), *__restrict__ R = cg(q.R), *__restrict__ C = cg(q.C);
-    __shared__ double Cs[GJB][GJB + 1];
-    __shared__ double Bs[GJB][GJB + 1];
+    __shared__ double Cs[GJB * SA], Bs[GJB * SB];
     const int r0 = ti * GJB, c0 = tj * GJB;
     const int hr = std::min(GJB, nc - r0), hc = std::min(GJB, nc - c0);
-    const int rr = 4 * (threadIdx.x / 16), cc = 4 * (threadIdx.x % 16);
-    const int lr = threadIdx.x >> 2, lq = (threadIdx.x & 3) * 16;  // load mapping: 64 rows x 4 quarters
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, kk = lane >> 4;
     if (ti == k) {
         // pivot block row: A_KK = P, A_Kj = R_j
-        if (lr < b)
-            for (int c = lq; c < lq + 16 && c < hc; c++)
-                A[(int64_t)(k0 + lr) * nc + c0 + c] = tj == k ? P[lr * GJB + c] : R[(int64_t)lr * nc + c0 + c];
+        for (int r = w; r < b; r += 4)
+            if (lane < hc)
+                A[(int64_t)(k0 + r) * nc + c0 + lane] = tj == k ? P[r * GJB + lane] : R[(int64_t)r * nc + c0 + lane];
         return;
     }
-    if (lr < hr)
-        for (int c = lq; c < lq + 16 && c < b; c++) Cs[lr][c] = C[(int64_t)(r0 + lr) * GJB + c];
-    if (lr < b)
-        for (int c = lq; c < lq + 16 && c < hc; c++)
-            Bs[lr][c] = tj == k ? P[lr * GJB + c] : R[(int64_t)lr * nc + c0 + c];
-    __syncthreads();
-    double acc[4][4] = {};
-    for (int l = 0; l < b; l++) {
-        double cv[4], bv[4];
-        for (int s = 0; s < 4; s++) {
-            cv[s] = Cs[rr + s][l];
-            bv[s] = Bs[l][cc + s];
+    // the tile's old values are in flight while the operands are staged
+    double old[4][4];
+    for (int mt = 0; mt < 4; mt++)
+        for (int r = 0; r < 4; r++) {
+            const int row = 16 * mt + kk + 4 * r, col = 16 * w + m;
+            old[mt][r] = tj != k && row < hr && col < hc ? A[(int64_t)(r0 + row) * nc + c0 + col] : 0.0;
         }
-        for (int x = 0; x < 4; x++)
-            for (int y = 0; y < 4; y++) acc[x][y] = fma(cv[x], bv[y], acc[x][y]);
+#pragma unroll 4
+    for (int r = w; r < GJB; r += 4) {
+        Cs[r * SA + lane] = r < hr && lane < b ? C[(int64_t)(r0 + r) * GJB + lane] : 0.0;
+        Bs[r * SB + lane] = r < b && lane < hc ? (tj == k ? P[r * GJB + lane] : R[(int64_t)r * nc + c0 + lane]) : 0.0;
     }
-    for (int x = 0; x < 4; x++)
-        for (int y = 0; y < 4; y++) {
-            const int r = rr + x, c = cc + y;
-            if (r >= hr || c >= hc) continue;
-            auto *a = A + (int64_t)(r0 + r) * nc + c0 + c;
-            *a = tj == k ? -acc[x][y] : *a - acc[x][y];
+    __syncthreads();
+    f64x4c acc[4];
+    for (int mt = 0; mt < 4; mt++) acc[mt] = f64x4c{0.0, 0.0, 0.0, 0.0};
+    mm_tiles<4, 16>(Cs, Bs + 16 * w, lane, acc);
+    for (int mt = 0; mt < 4; mt++)
+        for (int r = 0; r < 4; r++) {
+            const int row = 16 * mt + kk + 4 * r, col = 16 * w + m;
+            if (row < hr && col < hc) A[(int64_t)(r0 + row) * nc + c0 + col] = old[mt][r] - acc[mt][r];
         }
 }
 
@@ -549,7 +615,7 @@ int amr_coarse_form(hipStream_t s, amr_model *const *ms, int n, AmrStaging &stg)
     if (!fl.empty()) hipLaunchKernelGGL(fix_diag_kernel, grid(fl.size()), dim3(256), 0, s, dj, wl(o_f));
     AMR_HIP(hipGetLastError());
     for (int k = 0; k < maxnt; k++) {
-        hipLaunchKernelGGL(gj_pivot_kernel, grid(pv[k].size()), dim3(1024), 0, s, dj, wl(o_pv[k]), k);
+        hipLaunchKernelGGL(gj_pivot_kernel, grid(pv[k].size()), dim3(256), 0, s, dj, wl(o_pv[k]), k);
         hipLaunchKernelGGL(gj_panel_kernel, grid(pn[k].size()), dim3(256), 0, s, dj, wl(o_pn[k]), k);
         hipLaunchKernelGGL(gj_update_kernel, grid(up[k].size()), dim3(256), 0, s, dj, wl(o_up[k]), k);
     }
