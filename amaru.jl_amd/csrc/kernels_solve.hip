@@ -963,16 +963,17 @@ __device__ inline void mf_sum_q(const SegDesc &d, int64_t nd, const int32_t b[8]
         const auto *f = gl(d.mff);
         const auto *fp = gl(d.fptr), *src = gl(d.mfsrc);
         const int32_t k1 = fp[nd + 1];
-        for (int32_t k = fp[nd] + 8; k < k1; k += 4) {
-            int32_t e[4];
+        // eight at a time: a corner node of tetrahedra has up to 24
+        for (int32_t k = fp[nd] + 8; k < k1; k += 8) {
+            int32_t e[8];
 #pragma unroll
-            for (int j = 0; j < 4; j++) e[j] = src[k + j < k1 ? k + j : k];
+            for (int j = 0; j < 8; j++) e[j] = src[k + j < k1 ? k + j : k];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < 8; j++)
 #pragma unroll
                 for (int c = 0; c < 3; c++) v[j][c] = f[e[j] + 64 * c];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < 8; j++)
 #pragma unroll
                 for (int c = 0; c < 3; c++) a[c] = k + j < k1 ? a[c] + v[j][c] : a[c];
         }
