@@ -230,10 +230,14 @@ __device__ inline double inv3_entry(const double *J, int k, double *det_out)
 //
 // One 64-lane workgroup per element.  Lane (ch, b) = lane ch*NN + b owns the
 // node blocks (a, b) for a in chunk ch (ACH consecutive row nodes) and keeps
-// their 9*ACH entries in registers across all IPs.  Per IP: 9 lanes build J
-// and its inverse, NN lanes build dN/dX (and /sqrt2) into LDS, one lane
-// evaluates calcD for plastic states, then every lane forms DB for its
-// column node (54 fma) and updates its blocks (36 fma per block).
+// their 9*ACH entries in registers across all IPs.  Per chunk of up to nine
+// IPs the lanes first form J, its inverse, calcD (plastic elements) and dN/dX
+// (and /sqrt2) of all the chunk's IPs at once into LDS, with a barrier after
+// each; then every lane forms, IP after IP without barriers, DB for its column
+// node (54 fma) and updates its blocks (36 fma per block).  The sums are those
+// of one IP at a time with five barriers each, the same bits; that took 261 us
+// on the 40x40x20 HEX8 footing (147 MB of Ke: 29 us) and 469 us on HEX20
+// 17x19x15 with 27 IPs, this 106 and 247.
 
 // Each kernel's body is a device function of its workgroup index, inlined
 // into the single-model kernel (the workgroup index is blockIdx.x) and into
@@ -246,21 +250,23 @@ ke_kernel_at(int64_t bid_, int64_t ne, const double *__restrict__ X, const int32
              double *__restrict__ Ke, int32_t *__restrict__ err)
 {
     constexpr int NCH = (NN + ACH - 1) / ACH;
+    constexpr int QC = NQ > 9 ? 9 : NQ;  // IPs per chunk
+    static_assert(NQ % QC == 0, "IP chunks");
     const int64_t e = bid_;
     const int lane = threadIdx.x;
     __shared__ double sC[NN * 3];
-    __shared__ double sJ[9], sInv[9], sCoef;
-    __shared__ double sG[NN * 6];
-    __shared__ double sD[36];
+    __shared__ double sJ[QC][9], sInv[QC][9], sCoef[QC];
+    __shared__ double sG[QC][NN * 6];
+    __shared__ double sD[QC][36];
     __shared__ int sBad;
 
     for (int i = lane; i < NN * 3; i += 64) sC[i] = X[(int64_t)conn[e * NN + i / 3] * 3 + i % 3];
     const AmrMat m = mats[emat[e]];
+    const bool elastic = all_elastic || m.kind == AMR_MAT_LE;
     if (lane == 0) {
         sBad = 0;
-        if (all_elastic || m.kind == AMR_MAT_LE) calc_De(m.p[0], m.p[1], sD);
+        if (elastic) calc_De(m.p[0], m.p[1], sD[0]);
     }
-    const bool elastic = all_elastic || m.kind == AMR_MAT_LE;
     const int b = lane % NN, ch = lane / NN;
     const bool active = lane < NN * NCH;
     double acc[ACH][9];
@@ -270,72 +276,89 @@ ke_kernel_at(int64_t bid_, int64_t ne, const double *__restrict__ X, const int32
         for (int s = 0; s < 9; s++) acc[i][s] = 0.0;
     __syncthreads();
 
-    for (int q = 0; q < NQ; q++) {
-        const double *dq = dNdR + q * NN * 3;
-        if (lane < 9) {
-            int i = lane / 3, j = lane % 3;
-            double a = 0.0;
-            for (int n = 0; n < NN; n++) a = fma(sC[n * 3 + i], dq[n * 3 + j], a);
-            sJ[lane] = a;
+    for (int q0 = 0; q0 < NQ; q0 += QC) {
+        // row i of J at IP q: three chains over the nodes
+        for (int t = lane; t < QC * 3; t += 64) {
+            const int qc = t / 3, i = t - 3 * qc;
+            const double *dq = dNdR + (q0 + qc) * NN * 3;
+            double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+#pragma unroll 4
+            for (int n = 0; n < NN; n++) {
+                const double x = sC[n * 3 + i];
+                a0 = fma(x, dq[n * 3], a0);
+                a1 = fma(x, dq[n * 3 + 1], a1);
+                a2 = fma(x, dq[n * 3 + 2], a2);
+            }
+            sJ[qc][i * 3] = a0;
+            sJ[qc][i * 3 + 1] = a1;
+            sJ[qc][i * 3 + 2] = a2;
+        }
+        if (!elastic && lane >= 64 - QC) {
+            const int qc = lane - (64 - QC);
+            double s14[AMR_NSTATE];
+            const int64_t ip = e * NQ + q0 + qc;
+            for (int f = 0; f < AMR_NSTATE; f++) s14[f] = st[f * nip + ip];
+            calc_D(m, s14, sD[qc]);
         }
         __syncthreads();
-        if (lane < 9) {
+        for (int t = lane; t < QC * 9; t += 64) {
+            const int qc = t / 9, k = t - 9 * qc;
             double det;
-            sInv[lane] = inv3_entry(sJ, lane, &det);
-            if (lane == 0) {
-                sCoef = det * wip[q];
+            sInv[qc][k] = inv3_entry(sJ[qc], k, &det);
+            if (k == 0) {
+                sCoef[qc] = det * wip[q0 + qc];
                 if (!(det > 0.0)) sBad = 1;
             }
-        } else if (lane == 32 && !elastic) {
-            double s14[AMR_NSTATE];
-            int64_t ip = e * NQ + q;
-            for (int f = 0; f < AMR_NSTATE; f++) s14[f] = st[f * nip + ip];
-            calc_D(m, s14, sD);
         }
         __syncthreads();
-        if (lane < NN) {
+        for (int t = lane; t < QC * NN; t += 64) {
+            const int qc = t / NN, n = t - NN * qc;
+            const double *dq = dNdR + ((q0 + qc) * NN + n) * 3;
             double g[3];
             for (int j = 0; j < 3; j++) {
                 double a = 0.0;
-                for (int i = 0; i < 3; i++) a = fma(dq[lane * 3 + i], sInv[i * 3 + j], a);
+                for (int i = 0; i < 3; i++) a = fma(dq[i], sInv[qc][i * 3 + j], a);
                 g[j] = a;
             }
-            sG[lane * 6 + 0] = g[0];
-            sG[lane * 6 + 1] = g[1];
-            sG[lane * 6 + 2] = g[2];
-            sG[lane * 6 + 3] = g[0] / SR2;
-            sG[lane * 6 + 4] = g[1] / SR2;
-            sG[lane * 6 + 5] = g[2] / SR2;
+            double *G = sG[qc] + n * 6;
+            for (int j = 0; j < 3; j++) {
+                G[j] = g[j];
+                G[3 + j] = g[j] / SR2;
+            }
         }
         __syncthreads();
         if (active) {
-            const double coef = sCoef;
-            const double gx = sG[b * 6], gy = sG[b * 6 + 1], gz = sG[b * 6 + 2];
-            const double hx = sG[b * 6 + 3], hy = sG[b * 6 + 4], hz = sG[b * 6 + 5];
-            double DB[6][3];
+#pragma unroll 1
+            for (int qc = 0; qc < QC; qc++) {
+                const double coef = sCoef[qc];
+                const double *D = sD[elastic ? 0 : qc], *G = sG[qc];
+                const double gx = G[b * 6], gy = G[b * 6 + 1], gz = G[b * 6 + 2];
+                const double hx = G[b * 6 + 3], hy = G[b * 6 + 4], hz = G[b * 6 + 5];
+                double DB[6][3];
 #pragma unroll
-            for (int k = 0; k < 6; k++) {
-                DB[k][0] = fma(sD[k * 6 + 5], hy, fma(sD[k * 6 + 4], hz, fma(sD[k * 6 + 0], gx, 0.0)));
-                DB[k][1] = fma(sD[k * 6 + 5], hx, fma(sD[k * 6 + 3], hz, fma(sD[k * 6 + 1], gy, 0.0)));
-                DB[k][2] = fma(sD[k * 6 + 4], hx, fma(sD[k * 6 + 3], hy, fma(sD[k * 6 + 2], gz, 0.0)));
-            }
+                for (int k = 0; k < 6; k++) {
+                    DB[k][0] = fma(D[k * 6 + 5], hy, fma(D[k * 6 + 4], hz, fma(D[k * 6 + 0], gx, 0.0)));
+                    DB[k][1] = fma(D[k * 6 + 5], hx, fma(D[k * 6 + 3], hz, fma(D[k * 6 + 1], gy, 0.0)));
+                    DB[k][2] = fma(D[k * 6 + 4], hx, fma(D[k * 6 + 3], hy, fma(D[k * 6 + 2], gz, 0.0)));
+                }
 #pragma unroll
-            for (int ia = 0; ia < ACH; ia++) {
-                const int a = ch * ACH + ia;
-                if (a < NN) {
-                    const double ax = sG[a * 6], ay = sG[a * 6 + 1], az = sG[a * 6 + 2];
-                    const double bx = sG[a * 6 + 3], by = sG[a * 6 + 4], bz = sG[a * 6 + 5];
+                for (int ia = 0; ia < ACH; ia++) {
+                    const int a = ch * ACH + ia;
+                    if (a < NN) {
+                        const double ax = G[a * 6], ay = G[a * 6 + 1], az = G[a * 6 + 2];
+                        const double bx = G[a * 6 + 3], by = G[a * 6 + 4], bz = G[a * 6 + 5];
 #pragma unroll
-                    for (int c = 0; c < 3; c++) {
-                        // row r=0 (x): B rows 0 (ax), 4 (bz), 5 (by)
-                        double t0 = fma(by, DB[5][c], fma(bz, DB[4][c], fma(ax, DB[0][c], 0.0)));
-                        // r=1 (y): rows 1 (ay), 3 (bz), 5 (bx)
-                        double t1 = fma(bx, DB[5][c], fma(bz, DB[3][c], fma(ay, DB[1][c], 0.0)));
-                        // r=2 (z): rows 2 (az), 3 (by), 4 (bx)
-                        double t2 = fma(bx, DB[4][c], fma(by, DB[3][c], fma(az, DB[2][c], 0.0)));
-                        acc[ia][0 * 3 + c] = fma(coef, t0, acc[ia][0 * 3 + c]);
-                        acc[ia][1 * 3 + c] = fma(coef, t1, acc[ia][1 * 3 + c]);
-                        acc[ia][2 * 3 + c] = fma(coef, t2, acc[ia][2 * 3 + c]);
+                        for (int c = 0; c < 3; c++) {
+                            // row r=0 (x): B rows 0 (ax), 4 (bz), 5 (by)
+                            double t0 = fma(by, DB[5][c], fma(bz, DB[4][c], fma(ax, DB[0][c], 0.0)));
+                            // r=1 (y): rows 1 (ay), 3 (bz), 5 (bx)
+                            double t1 = fma(bx, DB[5][c], fma(bz, DB[3][c], fma(ay, DB[1][c], 0.0)));
+                            // r=2 (z): rows 2 (az), 3 (by), 4 (bx)
+                            double t2 = fma(bx, DB[4][c], fma(by, DB[3][c], fma(az, DB[2][c], 0.0)));
+                            acc[ia][0 * 3 + c] = fma(coef, t0, acc[ia][0 * 3 + c]);
+                            acc[ia][1 * 3 + c] = fma(coef, t1, acc[ia][1 * 3 + c]);
+                            acc[ia][2 * 3 + c] = fma(coef, t2, acc[ia][2 * 3 + c]);
+                        }
                     }
                 }
             }
