@@ -32,6 +32,7 @@
 #include <cstring>
 
 #include "amr_internal.h"
+#include "wave_ops.h"
 
 namespace {
 
@@ -137,15 +138,11 @@ __device__ inline void reg_terms(double x, double y, double z, double *t)
     t[6] = x * z;
 }
 
-// Sum over the 64 lanes by an xor butterfly: every lane ends with the same
-// bits (each step adds the same two operands, in either order).
-__device__ inline double wave_sum(double x)
-{
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o, 64);
-    return x;
-}
 
+// Bound by the sums over the wave, up to 25 in each of seven dependent steps:
+// with shuffles (an LDS round trip per level) 384 us for the 6,480 patches of
+// a HEX20 21x19x20 block, with DPP moves (wave_sum) 224 us.
+//
 // One 64-lane wave per patch.  Lane l holds rows l, l+64, l+128, l+192 of
 // the patch's matrix [basis | IP values] (m x NCOL) in registers; each
 // Householder step reduces the reflector's norm and its products with the
