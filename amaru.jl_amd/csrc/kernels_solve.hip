@@ -24,7 +24,8 @@
 // the scalar sums those partials itself in index order (kernel boundaries
 // make them visible).
 //
-// Precision.  Plain path: FP64 PCG.  Mixed paths: the same CG recurrences
+// Precision.  Matrix-free members (all-elastic models) multiply in FP64 from
+// the element geometry in every mode.  Plain path: FP64 PCG.  Mixed paths: the same CG recurrences
 // with FP64 vectors, FP64 dot products and FP64 solution update, but the
 // SpMV reads FP32 values (with an FP32 copy of the search direction and FP32
 // accumulation for AMR_PREC_MIXED, FP64 gather and accumulation for
@@ -337,9 +338,11 @@ __device__ inline int64_t block_col<int16_t>(const int16_t *__restrict__ col, in
     return row + gl(col)[k];
 }
 
-template <int L, bool ABS, typename VT, typename XT, typename AT, typename CT = int32_t>
+// FUSE: the operand is z + beta x, formed as it is gathered.
+template <int L, bool ABS, typename VT, typename XT, typename AT, typename CT = int32_t, bool FUSE = false>
 __device__ inline void row_sum(int32_t rb, int32_t re, int sub, const CT *__restrict__ col,
-                               const VT *__restrict__ vals, const XT *__restrict__ x, AT y[3], int64_t row = 0)
+                               const VT *__restrict__ vals, const XT *__restrict__ x, AT y[3], int64_t row = 0,
+                               const double *__restrict__ z = nullptr, double beta = 0.0)
 {
     constexpr int NS = 64 / L;
     AT acc[NS][3];
@@ -352,7 +355,13 @@ __device__ inline void row_sum(int32_t rb, int32_t re, int sub, const CT *__rest
             if (k < re) {
                 const int64_t c = block_col<CT>(col, k, row);
                 const auto *xc = gl(x) + c * 3;
-                const AT x0 = (AT)xc[0], x1 = (AT)xc[1], x2 = (AT)xc[2];
+                AT x0 = (AT)xc[0], x1 = (AT)xc[1], x2 = (AT)xc[2];
+                if (FUSE) {
+                    const auto *zc = gl(z) + c * 3;
+                    x0 = fma(beta, x0, zc[0]);
+                    x1 = fma(beta, x1, zc[1]);
+                    x2 = fma(beta, x2, zc[2]);
+                }
                 AT v[9];
                 load_block<VT, AT>(vals, k, v);
                 if (ABS) {
@@ -615,8 +624,10 @@ __global__ void __launch_bounds__(WGS) residual_kernel(const SegDesc *__restrict
 
 // ------------------------------------------------------------------- PCG
 //
-// Iteration k of a model (parity pi = k % 2), three kernels:
-//   pcg_spmv:   q = A p, partial p.q                          -> P_PQ
+// Iteration k of a model (parity pi = k % 2), three kernels; without a coarse
+// correction the first forms the direction as it gathers (matrix-free members
+// and small assembled ones) and pcg_dir is not launched:
+//   pcg_spmv / pcg_mf: q = A p, partial p.q                   -> P_PQ
 //   pcg_update: a = rz_k / pq; x += a p; r -= a q; z = M r;
 //               partials rz_{k+1}, rr                         -> P_RZ[pi], P_RR[pi]
 //   pcg_dir:    b = rz_{k+1} / rz_k; p = z + b p; convergence test;
@@ -637,8 +648,13 @@ __device__ inline const double *seg_px<double>(const SegDesc &d) { return d.p; }
 template <>
 __device__ inline const float *seg_px<float>(const SegDesc &d) { return d.p32; }
 
-template <int L, typename VT, typename XT, typename AT>
-__global__ void __launch_bounds__(WGS) pcg_spmv_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ tl)
+// FUSE (small models without a coarse correction): the kernel gathers
+// p = z + beta p as pcg_mf_kernel does, with its bookkeeping; pcg_update stores
+// it.  For the gather's second vector an iteration saves the direction's
+// launch (about 5 us).
+template <int L, typename VT, typename XT, typename AT, bool FUSE>
+__global__ void __launch_bounds__(WGS) pcg_spmv_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ tl,
+                                                       int first)
 {
     const int2 te = list_entry(tl, xcd_tile(blockIdx.x, gridDim.x));
     if (te.x < 0) return;  // padding of a captured step's list
@@ -651,7 +667,29 @@ __global__ void __launch_bounds__(WGS) pcg_spmv_kernel(const SegDesc *__restrict
         if (te.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
         return;
     }
-    if (te.y == 0 && threadIdx.x == 0) ctl[C_ITERS] = ctl[C_ITERS] + 1;
+    // the step's first iteration takes p as it is: p + 0 p
+    const double *z = FUSE && !first ? d.z : d.p;
+    double beta = 0.0;
+    if (FUSE && !first) {
+        const int it = ctl[C_PREV], pi = (it - 1) & 1;
+        const double rzt = thread_partials<WGS>(d.part + (pi ? P_RZ1 : P_RZ0), d.nred);
+        const double rrt = te.y == 0 ? thread_partials<WGS>(d.part + (pi ? P_RR1 : P_RR0), d.nred) : 0.0;
+        const double rzn = block_sum<WGS>(rzt);
+        beta = rzn / glw(d.scal)[rz_pub(1 - pi)];
+        if (te.y == 0) {
+            const double rr = block_sum<WGS>(rrt);
+            if (threadIdx.x == 0) {
+                glw(d.scal)[S_RR] = rr;
+                glw(d.scal)[S_RZ] = rzn;
+                glw(d.scal)[rz_pub(pi)] = rzn;
+                glw(d.scal)[S_BETA] = beta;
+                if (rr <= glw(d.scal)[S_THR] || it >= d.maxiter || !std::isfinite(rr)) ctl[C_STOP] = 1;
+                else ctl[C_ITERS] = it + 1;
+            }
+        }
+    } else if (te.y == 0 && threadIdx.x == 0) {
+        ctl[C_ITERS] = (FUSE ? ctl[C_PREV] : ctl[C_ITERS]) + 1;
+    }
     const int R = d.R;
     extern __shared__ __align__(16) char sm[];
     int32_t *srp = tile_rowptr(sm);
@@ -673,12 +711,13 @@ __global__ void __launch_bounds__(WGS) pcg_spmv_kernel(const SegDesc *__restrict
         if (sub < 3) {
             mk = gl(d.mask)[k3];
             pk = gl(d.p)[k3];
+            if (FUSE) pk = fma(beta, pk, gl(z)[k3]);
         }
         AT y[3];
         if (d.col16)
-            row_sum<L, false, VT, XT, AT, int16_t>(srp[i], srp[i + 1], sub, d.col16, vals, px, y, r0 + i);
+            row_sum<L, false, VT, XT, AT, int16_t, FUSE>(srp[i], srp[i + 1], sub, d.col16, vals, px, y, r0 + i, z, beta);
         else
-            row_sum<L, false, VT, XT, AT>(srp[i], srp[i + 1], sub, d.col, vals, px, y);
+            row_sum<L, false, VT, XT, AT, int32_t, FUSE>(srp[i], srp[i + 1], sub, d.col, vals, px, y, 0, z, beta);
         // lane e < 3 stores q of component e; lane 0 forms the row's p.q,
         // fma(p2, q2, fma(p1, q1, fma(p0, q0, 0)))
         const double qk = mk != 0.0 ? (double)(sub == 0 ? y[0] : sub == 1 ? y[1] : y[2]) : 0.0;
@@ -987,7 +1026,8 @@ __device__ inline void mf_sum_q(const SegDesc &d, int64_t nd, const int32_t b[8]
 // writes the chunk's part of c = Phi^T r, while r is in registers (a kernel of
 // its own for it read r and X again: 3.7 us of a 36 us iteration on the
 // 40x40x20 footing).
-template <bool MF, bool TL>
+// FZ: members on an assembled matrix whose SpMV forms the direction.
+template <bool MF, bool TL, bool FZ>
 __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl,
                                                          int first)
 {
@@ -995,15 +1035,16 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
     if (ve.x < 0) return;
     const SegDesc d = D[ve.x];
     auto *ctl = glw(d.ctl);
-    const bool fuse = MF && d.fuse && !first;
-    const int done = ctl[C_DONE], stop = MF ? (int)ctl[C_STOP] : 0, iters = ctl[C_ITERS];
+    constexpr bool FUSE = MF || FZ;  // the operator may form the direction
+    const bool fuse = FUSE && d.fuse && !first;
+    const int done = ctl[C_DONE], stop = FUSE ? (int)ctl[C_STOP] : 0, iters = ctl[C_ITERS];
     const int pi = (iters - 1) & 1;
     auto *__restrict__ x = glw(d.x);
     auto *__restrict__ r = glw(d.r);
     auto *__restrict__ z = glw(d.z);
     auto *__restrict__ p = glw(d.p);
     const auto *__restrict__ q = gl(d.q);
-    const double beta = MF ? (double)glw(d.scal)[S_BETA] : 0.0;
+    const double beta = FUSE ? (double)glw(d.scal)[S_BETA] : 0.0;
     const double rzp0 = glw(d.scal)[S_RZP0], rzp1 = glw(d.scal)[S_RZP1];
     // z is read where the direction is formed here (else p again, unused, so
     // that the loads need no branch)
@@ -1017,7 +1058,7 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
     auto load_node = [&](int64_t n, Node &v) {
         for (int c = 0; c < 3; c++) {
             v.p[c] = p[n * 3 + c];
-            if (MF) v.z[c] = zs[n * 3 + c];
+            if (FUSE) v.z[c] = zs[n * 3 + c];
             v.x[c] = x[n * 3 + c];
             v.r[c] = r[n * 3 + c];
             if (MF) v.m[c] = gl(d.mask)[n * 3 + c];
@@ -1047,12 +1088,12 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
     load_node(nd, v);
     AMR_ISSUED();
     if (done) return;
-    if (MF && stop) {
+    if (FUSE && stop) {
         // converged before this iteration (seen by the operator's first tile)
         if (ve.y == 0 && threadIdx.x == 0) ctl[C_DONE] = 1;
         return;
     }
-    if (MF && ve.y == 0 && threadIdx.x == 0) ctl[C_PREV] = iters;
+    if (FUSE && ve.y == 0 && threadIdx.x == 0) ctl[C_PREV] = iters;
     double fv[8][3];
     if (MF) mf_load_q(d, v.b, fv);
     const double pqt = thread_partials<WGV>(d.part + P_PQ, d.npq);
@@ -1525,7 +1566,8 @@ size_t tile_lds(int R, int ndbl) { return (size_t)(((R + 1) * 4 + 15) & ~15) + (
 enum { K_F64 = 0, K_F32, K_F32D, K_NKIND };
 // Launch groups after those: the matrix-free operator of each element shape,
 // with one wave per group and with shared groups
-enum { K_MF = K_NKIND, K_NGROUP = K_NKIND + 8 };
+enum { K_MF = K_NKIND, K_FZ = K_MF + 8, K_NGROUP = K_FZ + 2 };
+// K_FZ: the SpMV that forms the direction, FP64 values; + 1: FP32 values
 
 int lanes_index(int lanes) { return lanes == 8 ? 0 : lanes == 16 ? 1 : lanes == 32 ? 2 : 3; }
 constexpr int LANES[4] = {8, 16, 32, 64};
@@ -1535,16 +1577,19 @@ int kind_lanes(const amr_model *m, int kind)
     return kind == K_F64 ? m->lanes64 : kind == K_F32 ? m->lanes32 : m->lanes32d;
 }
 
-void launch_pcg_spmv(int kind, int lanes, unsigned grid, int Rmax, hipStream_t s, const SegDesc *D, const int2 *tl)
+void launch_pcg_spmv(int kind, int lanes, unsigned grid, int Rmax, hipStream_t s, const SegDesc *D, const int2 *tl,
+                     int first)
 {
     const size_t lds = tile_lds(Rmax, 1);
-#define AMR_PCG_SPMV(LN, VT, XT, AT) \
-    hipLaunchKernelGGL((pcg_spmv_kernel<LN, VT, XT, AT>), dim3(grid), dim3(WGS), lds, s, D, tl)
-#define AMR_PCG_KIND(LN)                                          \
-    do {                                                          \
-        if (kind == K_F64) AMR_PCG_SPMV(LN, double, double, double); \
-        else if (kind == K_F32) AMR_PCG_SPMV(LN, float, float, float); \
-        else AMR_PCG_SPMV(LN, float, double, double);             \
+#define AMR_PCG_SPMV(LN, VT, XT, AT, FZ) \
+    hipLaunchKernelGGL((pcg_spmv_kernel<LN, VT, XT, AT, FZ>), dim3(grid), dim3(WGS), lds, s, D, tl, first)
+#define AMR_PCG_KIND(LN)                                                     \
+    do {                                                                     \
+        if (kind == K_F64) AMR_PCG_SPMV(LN, double, double, double, false);  \
+        else if (kind == K_F32) AMR_PCG_SPMV(LN, float, float, float, false); \
+        else if (kind == K_F32D) AMR_PCG_SPMV(LN, float, double, double, false); \
+        else if (kind == K_FZ) AMR_PCG_SPMV(LN, double, double, double, true); \
+        else AMR_PCG_SPMV(LN, float, double, double, true);                  \
     } while (0)
     switch (lanes) {
     case 8: AMR_PCG_KIND(8); break;
@@ -1765,6 +1810,13 @@ int handoff(amr_model *m, hipStream_t from, hipStream_t to)
     return AMR_OK;
 }
 
+// Members on an assembled matrix without a coarse correction: up to this many
+// nodes the direction is formed in the SpMV's gather (a launch less per
+// iteration).  Passes with and without: HEX20 31x4x5 dynamic (3,400 nodes) 97.1
+// and 100.3 ms, TET10 20x5x5 von Mises (5,000) 25.0 and 25.9, HEX8 64x16x16
+// (18,800) 12.9 and 13.5, HEX20 40x10x10 with 27 IPs (20,000) 39.7 and 39.1.
+constexpr int64_t FUSE_MAX = 16384;
+
 // Two-level members on an assembled matrix: the update kernel by chunks, with
 // the restriction.  On the matrix-free operator it stays in node order: summing
 // the elements' products in aggregate order lost more (TET10 49x12x13: 13.3 ->
@@ -1836,6 +1888,7 @@ void fill_desc(amr_pool *p, int slot)
         d.nchunk = m->nchunk;
         set_cparts(d, !M.mf);
     }
+    if (!d.tl && !(M.mixed && M.f32x) && m->nnodes <= FUSE_MAX) d.fuse = 1;
     if (M.mf) {
         const MfGeom mg = mf_geom(m);
         d.geo = m->mf_geo;
@@ -1913,8 +1966,9 @@ void build_groups(amr_pool *p, const std::vector<int> &slots, bool residual, std
             continue;
         }
         const int kind = residual ? K_F64 : member_kind(M);
-        const int key = kind * 4 + lanes_index(kind_lanes(M.m, kind));
         const SegDesc &d = p->hD[s];
+        const int gk = !residual && d.fuse ? K_FZ + (kind == K_F32D ? 1 : 0) : kind;
+        const int key = gk * 4 + lanes_index(kind_lanes(M.m, kind));
         for (int t = 0; t < d.ntiles; t++) ent[key].push_back(make_int2(s, t));
         rmax[key] = std::max(rmax[key], d.R);
     }
@@ -2265,11 +2319,11 @@ int amr_pool_step_launch(amr_pool *p)
     // direction kernels for the one-level members that have one in every
     // iteration (vd), for all of them in the step's last one (vl), and for
     // the two-level members (vt)
-    enum { V_M, V_A, V_AT, V_RS, V_D, V_L, V_T, V_CW, NV };
+    enum { V_M, V_A, V_AF, V_AT, V_RS, V_D, V_L, V_T, V_CW, NV };
     std::vector<int> sv[NV];
     for (int s : act) {
         const SegDesc &d = p->hD[s];
-        sv[p->mem[s].mf ? V_M : d.tl ? V_AT : V_A].push_back(s);
+        sv[p->mem[s].mf ? V_M : d.tl ? V_AT : d.fuse ? V_AF : V_A].push_back(s);
         if (d.tl && p->mem[s].mf) sv[V_RS].push_back(s);
         if (!d.tl) {
             sv[V_L].push_back(s);
@@ -2286,7 +2340,9 @@ int amr_pool_step_launch(amr_pool *p)
         const Member &M = p->mem[act[0]];
         const int kind = member_kind(M);
         if (M.mf) gr.push_back({mf_kind(M.m), 0, 0, 0, (unsigned)d.npq});
-        else gr.push_back({kind, kind_lanes(M.m, kind), d.R, 0, (unsigned)d.ntiles});
+        else
+            gr.push_back({d.fuse ? K_FZ + (kind == K_F32D ? 1 : 0) : kind, kind_lanes(M.m, kind), d.R, 0,
+                          (unsigned)d.ntiles});
     } else {
         build_groups(p, act, false, ent, gr);
         for (int k = 0; k < NV; k++)
@@ -2351,17 +2407,18 @@ int amr_pool_step_launch(amr_pool *p)
             // the previous step formed it)
             const int first = j == 0 ? 1 : 0;
             for (const Group &g : gr) {
-                if (g.kind >= K_MF) launch_pcg_mf(g.kind, g.n, st, D, list(g.off), first);
-                else launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, D, list(g.off));
+                if (g.kind >= K_MF && g.kind < K_FZ) launch_pcg_mf(g.kind, g.n, st, D, list(g.off), first);
+                else launch_pcg_spmv(g.kind, g.lanes, g.n, g.Rmax, st, D, list(g.off), first);
             }
             if (p->timing) (void)hipEventRecord(p->ev[2 * j + 1], st);
             auto launch = [&](int k, auto kernel, int threads, auto... args) {
                 if (nv[k])
                     hipLaunchKernelGGL(kernel, dim3(nv[k]), dim3(threads), 0, st, D, list(o_v[k]), args...);
             };
-            launch(V_M, pcg_update_kernel<true, false>, WGV, first);
-            launch(V_A, pcg_update_kernel<false, false>, WGV, first);
-            launch(V_AT, pcg_update_kernel<false, true>, WGV, first);
+            launch(V_M, pcg_update_kernel<true, false, false>, WGV, first);
+            launch(V_A, pcg_update_kernel<false, false, false>, WGV, first);
+            launch(V_AF, pcg_update_kernel<false, false, true>, WGV, first);
+            launch(V_AT, pcg_update_kernel<false, true, false>, WGV, first);
             launch(V_RS, tl_restrict_kernel, 64, 0);
             launch(V_CW, tl_coarse_kernel, 256, 0);
             launch(j == check - 1 ? V_L : V_D, pcg_dir_kernel<false>, WGV);
@@ -2372,7 +2429,7 @@ int amr_pool_step_launch(amr_pool *p)
     // them: one each kernel by kernel, one graph launch when captured
     auto has = [&](int k) { return (int64_t)(nv[k] ? 1 : 0); };
     const int64_t iter_kernels =
-        (int64_t)check * ((int64_t)gr.size() + has(V_M) + has(V_A) + has(V_AT) + has(V_RS) + has(V_CW) + has(V_T)) +
+        (int64_t)check * ((int64_t)gr.size() + has(V_M) + has(V_A) + has(V_AF) + has(V_AT) + has(V_RS) + has(V_CW) + has(V_T)) +
         (check - 1) * has(V_D) + has(V_L);
     p->iter_kernels += iter_kernels;
     p->iter_submits += graph ? 1 : iter_kernels;
@@ -2561,7 +2618,7 @@ int step_decide(amr_pool *p, std::vector<amr_pool_result> &out)
             d.wp32 = wp32;
             if (!M.mf) {
                 d.geo = nullptr;
-                d.fuse = 0;
+                d.fuse = !d.tl && M.m->nnodes <= FUSE_MAX ? 1 : 0;
                 d.npq = d.ntiles;
                 if (d.tl) set_cparts(d, true);
             }
@@ -2795,10 +2852,10 @@ int amr_tune_lanes(amr_model *m)
         float best = 1e30f;
         int bestL = 64;
         for (int L : LANES) {
-            launch_pcg_spmv(kind, L, (unsigned)g.ntiles, g.R, p->stream, p->dD, Ls.dev_at<int2>(o));  // warm
+            launch_pcg_spmv(kind, L, (unsigned)g.ntiles, g.R, p->stream, p->dD, Ls.dev_at<int2>(o), 1);  // warm
             AMR_HIP(hipEventRecord(e0, p->stream));
             for (int rep = 0; rep < 3; rep++)
-                launch_pcg_spmv(kind, L, (unsigned)g.ntiles, g.R, p->stream, p->dD, Ls.dev_at<int2>(o));
+                launch_pcg_spmv(kind, L, (unsigned)g.ntiles, g.R, p->stream, p->dD, Ls.dev_at<int2>(o), 1);
             AMR_HIP(hipEventRecord(e1, p->stream));
             AMR_HIP(hipEventSynchronize(e1));
             float ms = 0.f;
