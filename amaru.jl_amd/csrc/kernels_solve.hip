@@ -1253,12 +1253,13 @@ __global__ void __launch_bounds__(WGV) pcg_dir_kernel(const SegDesc *__restrict_
 
 // Two-level pieces, for the members with d.tl (mode 0: inside the iteration,
 // skipped once the member is done; mode 1: initialisation and resume)
-//   restrict: c_a = sum_{i in a} R_i^T r_i, one wave per aggregate (inside an
-//             iteration only for the members whose update kernel does not
+//   restrict: c_a = sum_{i in a} R_i^T r_i, four waves per aggregate (inside
+//             an iteration only for the members whose update kernel does not
 //             write c's parts)
 //   coarse:   y = Kc^-1 c, one wave per coarse row, and partials of c.y
 //   prolong:  p = z + Phi y (start of a search direction)
-__global__ void __launch_bounds__(64) tl_restrict_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ al,
+constexpr int WGR = 256;  // restriction
+__global__ void __launch_bounds__(WGR) tl_restrict_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ al,
                                                          int mode)
 {
     const int2 e = list_entry(al, blockIdx.x);
@@ -1270,16 +1271,18 @@ __global__ void __launch_bounds__(64) tl_restrict_kernel(const SegDesc *__restri
     const auto *aggptr = gl(d.aggptr), *aggnodes = gl(d.aggnodes);
     const double cx = cent[a * 3], cy = cent[a * 3 + 1], cz = cent[a * 3 + 2];
     double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    // a lane's nodes k = k0 + lane + 64 j in order of j, eight at a time:
-    // the eight nodes' loads are issued before their sums
+    // a thread's nodes k = k0 + tid + 256 j in order of j, eight at a time:
+    // the eight nodes' loads are issued before their sums.  Bound by that chain
+    // of loads: on 256 aggregates of 1,057 nodes one wave each took 9.9 us, four
+    // take 6.6; with 261 nodes in each a TET10 step went from 7.43 to 7.30 ms
     constexpr int NB = 8;
     const int32_t k0 = aggptr[a], k1 = aggptr[a + 1];
     AMR_ISSUED();
     if (done) return;
-    for (int32_t kb = k0 + threadIdx.x; kb < k1; kb += 64 * NB) {
+    for (int32_t kb = k0 + (int32_t)threadIdx.x; kb < k1; kb += WGR * NB) {
         int64_t nd[NB];
 #pragma unroll
-        for (int j = 0; j < NB; j++) nd[j] = kb + 64 * j < k1 ? aggnodes[kb + 64 * j] : -1;
+        for (int j = 0; j < NB; j++) nd[j] = kb + WGR * j < k1 ? aggnodes[kb + WGR * j] : -1;
         double r[NB][3], x[NB][3];
 #pragma unroll
         for (int j = 0; j < NB; j++)
@@ -1301,10 +1304,14 @@ __global__ void __launch_bounds__(64) tl_restrict_kernel(const SegDesc *__restri
                 v[5] += fma(dx, r1, -dy * r0);
             }
     }
-    for (int q = 0; q < 6; q++)
-        for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_down(v[q], off, 64);
-    if (threadIdx.x == 0)
-        for (int q = 0; q < 6; q++) glw(d.cvec)[a * 6 + q] = v[q];
+    __shared__ double s[6][WGR / 64];
+    for (int q = 0; q < 6; q++) {
+        const double t = wave_sum(v[q]);
+        if (threadIdx.x % 64 == 0) s[q][threadIdx.x / 64] = t;
+    }
+    __syncthreads();
+    const int q = threadIdx.x;
+    if (q < 6) glw(d.cvec)[a * 6 + q] = (s[q][0] + s[q][1]) + (s[q][2] + s[q][3]);
 }
 
 __global__ void __launch_bounds__(256) tl_coarse_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ wl,
@@ -1938,7 +1945,7 @@ void launch_tl_fresh(amr_pool *p, const Lists &Ls, size_t o_al, unsigned nal, si
                      size_t o_pv, unsigned npv)
 {
     hipStream_t st = p->stream;
-    if (nal) hipLaunchKernelGGL(tl_restrict_kernel, dim3(nal), dim3(64), 0, st, p->dD, Ls.dev_at<int2>(o_al), 1);
+    if (nal) hipLaunchKernelGGL(tl_restrict_kernel, dim3(nal), dim3(WGR), 0, st, p->dD, Ls.dev_at<int2>(o_al), 1);
     if (ncw) hipLaunchKernelGGL(tl_coarse_kernel, dim3(ncw), dim3(256), 0, st, p->dD, Ls.dev_at<int2>(o_cw), 1);
     if (npv) hipLaunchKernelGGL(tl_prolong_kernel, dim3(npv), dim3(WGV), 0, st, p->dD, Ls.dev_at<int2>(o_pv));
 }
@@ -2419,7 +2426,7 @@ int amr_pool_step_launch(amr_pool *p)
             launch(V_A, pcg_update_kernel<false, false, false>, WGV, first);
             launch(V_AF, pcg_update_kernel<false, false, true>, WGV, first);
             launch(V_AT, pcg_update_kernel<false, true, false>, WGV, first);
-            launch(V_RS, tl_restrict_kernel, 64, 0);
+            launch(V_RS, tl_restrict_kernel, WGR, 0);
             launch(V_CW, tl_coarse_kernel, 256, 0);
             launch(j == check - 1 ? V_L : V_D, pcg_dir_kernel<false>, WGV);
             launch(V_T, pcg_dir_kernel<true>, WGV);

@@ -41,3 +41,32 @@ def test_chunks_match_direct(amaru, plastic, target, precision):
     assert np.linalg.norm(U - Uo) <= 1e-8 * np.linalg.norm(Uo)
     assert np.linalg.norm(F - Fo) <= 1e-8 * np.linalg.norm(Fo)
     dev.close()
+
+
+@pytest.mark.parametrize("target", [3, 64, 256, 257, 1100, 100000])
+def test_restrictions_agree(amaru, target):
+    """The restriction's own kernel (elastic models) against the chunks of the
+    update kernel (Drucker-Prager, not yet plastic: the same K), with
+    aggregates below, at and above a workgroup's 256 nodes and, at the last,
+    above the 2,048 it holds in flight.  The two iterations differ by rounding
+    only, so their lengths differ by a few iterations at most; a node left out
+    of a restriction costs many."""
+    am = amaru
+    mesh = am.Mesh(am.Block([[0, 0, 0], [2.0, 1.0, 1.0]], nx=19, ny=11, nz=10, cellshape="HEX8"))
+    its, Us = [], []
+    for mat in (am.LinearElastic(E=50e6, nu=0.3),
+                am.DruckerPrager(E=50e6, nu=0.3, alpha=0.23094, kappa=24000.0, H=0.0)):
+        model = am.FEModel(mesh, [("all", am.MechSolid, mat)])
+        bcs = [("x==0", am.SurfaceBC(ux=0, uy=0, uz=0)), ("x==2", am.SurfaceBC(tz=-1e3))]
+        model.configure_dofs(bcs)
+        U, F = model.bc_vals(bcs)
+        dev = am.DeviceModel(model)
+        dev.set_coarse(target)
+        dev.assemble()
+        r = dev.solve_system(U, F, rtol=1e-10, precond="two_level")
+        assert r["converged"]
+        its.append(r["iterations"])
+        Us.append(U)
+        dev.close()
+    assert abs(its[0] - its[1]) <= 4, its
+    assert np.linalg.norm(Us[0] - Us[1]) <= 1e-8 * np.linalg.norm(Us[1])
