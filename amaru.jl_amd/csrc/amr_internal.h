@@ -241,7 +241,15 @@ struct amr_model {
     int32_t *mf_conn = nullptr, *mf_src = nullptr, *mf_rec = nullptr, *mf_flag = nullptr;
     char *mf_block = nullptr;       // the arrays above are slices of it
     std::vector<double> mf_tab_h;   // host copy of mf_tab while it is uploaded
+    // set by tests only (amr_test_early_stops)
+    int test_early = 0;
+    double test_early_rtol = 0.0;
 };
+
+// For tests, not part of the public interface: the recursion of the model's
+// later solves stops n times too early, the k-th time (from 1) at rtol^k of
+// |b|, so that the check of the true residual refuses the stop (n = 0: off).
+extern "C" int amr_test_early_stops(amr_model *m, int n, double rtol);
 
 enum { SV_UEX = 0, SV_FEX, SV_U, SV_F, SV_DFEX, SV_R, SV_RC, SV_DUA, SV_DUI, SV_DFIN, SV_DUT, SV_X };
 

@@ -1425,14 +1425,23 @@ __global__ void __launch_bounds__(WGV) pcg_init_kernel(const SegDesc *__restrict
     }
 }
 
-// r = rt; z = M r; with restart also p = z (the search direction starts
-// afresh); rz partials into the slot the next iteration reads as "previous".
+// r = rt; z = M r; rz partials into the slot the next iteration reads as
+// "previous".  The search direction the next iteration takes as it is:
+//   REZ_KEEP     already in p (pcg_dir_kernel formed it)
+//   REZ_RESTART  p = z: it starts afresh
+//   REZ_FORM     p = z + beta p with the z and beta of the stop: a member whose
+//                operator forms the direction (d.fuse) stopped inside a step,
+//                before anything stored it; p still is the direction of the
+//                iteration before, orthogonal to r, and no later iteration
+//                would leave that state
+enum { REZ_KEEP = 0, REZ_RESTART, REZ_FORM, REZ_NMODE };
 __global__ void __launch_bounds__(WGV) pcg_rez_kernel(const SegDesc *__restrict__ D, const int2 *__restrict__ vl,
-                                                      int restart)
+                                                      int mode)
 {
     const int2 ve = vl[blockIdx.x];
     const SegDesc &d = D[ve.x];
     const int slot_pi = 1 - (glw(d.ctl)[C_ITERS] & 1);
+    const double beta = d.scal[S_BETA];
     float *__restrict__ p32 = d.wp32 ? d.p32 : nullptr;
     double rz = 0.0;
     const int64_t stride = (int64_t)d.nvblk * WGV;
@@ -1442,9 +1451,10 @@ __global__ void __launch_bounds__(WGV) pcg_rez_kernel(const SegDesc *__restrict_
         apply_prec(d, nd, rv, zv);
         for (int c = 0; c < 3; c++) {
             const int64_t i = nd * 3 + c;
+            if (mode == REZ_FORM) d.p[i] = fma(beta, d.p[i], d.z[i]);
             d.r[i] = rv[c];
             d.z[i] = zv[c];
-            if (restart) {
+            if (mode == REZ_RESTART) {
                 d.p[i] = zv[c];
                 if (p32) p32[i] = (float)zv[c];
             }
@@ -1663,7 +1673,9 @@ struct Member {
     bool form = false;  // its coarse operator is to be formed before it starts
     // per-step scratch
     bool rep = false, done = false;
+    bool unformed = false;  // stopped before its next direction was stored (REZ_FORM)
     double rr_rec = 0.0;
+    int early = 0;  // early stops still to come (amr_test_early_stops)
 };
 
 // M_WAIT: joined, but work the model queued on its own stream before
@@ -1835,6 +1847,16 @@ void set_cparts(SegDesc &d, bool on)
     d.nred = on ? d.nchunk : d.nvblk;
 }
 
+// The recursion stops where |r|^2 falls to this times |b|^2: half the
+// tolerance, or, for the early stops a test asks for, the next power of
+// early_rtol.
+double stop_factor(const Member &M)
+{
+    const double rtol = M.early > 0 ? std::pow(M.m->test_early_rtol, M.m->test_early - M.early + 1) : M.o.rtol;
+    const double tr = 0.5 * rtol;
+    return tr * tr;
+}
+
 void fill_desc(amr_pool *p, int slot)
 {
     Member &M = p->mem[slot];
@@ -1865,8 +1887,7 @@ void fill_desc(amr_pool *p, int slot)
     d.ctl = (int32_t *)(d.scal + S_NSCAL);
     d.nnodes = m->nnodes;
     d.nblk = m->pat.nblk;
-    const double tr = 0.5 * M.o.rtol;
-    d.thr_fac = tr * tr;
+    d.thr_fac = stop_factor(M);
     d.R = g.R;
     d.ntiles = g.ntiles;
     d.nvblk = g.nvblk;
@@ -2215,6 +2236,7 @@ int amr_pool_join(amr_pool *p, amr_model *m, const double *b, double *x, const a
     M.mf = m->mf_ok && m->mf_plain;
     M.mixed = M.pc32 && !M.mf;
     M.f32x = o->precision == AMR_PREC_MIXED;
+    M.early = m->test_early;
     if (int rc = pool_begin_host_writes(p)) return rc;
     // the model's queued work (assembly, right-hand side) precedes its solve
     if (m->stream != p->stream) {
@@ -2531,6 +2553,8 @@ int step_decide(amr_pool *p, std::vector<amr_pool_result> &out)
         M.iters = hc[C_ITERS];
         M.broke = hc[C_BREAK];
         M.done = hc[C_DONE] != 0 || hc[C_STOP] != 0;
+        // (after a step's last iteration pcg_dir_kernel forms it)
+        M.unformed = p->hD[s].fuse && M.done && !M.broke && M.iters - prev < check;
         const double rr = hs[S_RR];
         const double ratio = M.o.replace_ratio > 0.0 ? M.o.replace_ratio : 0.1;
         // mixed: replace when the recursive residual fell by `ratio`, and
@@ -2579,7 +2603,8 @@ int step_decide(amr_pool *p, std::vector<amr_pool_result> &out)
     AMR_HIP(hipMemcpyAsync(p->hS, p->dS, sbytes, hipMemcpyDeviceToHost, st));
     if (int rc = pool_sync(p)) return rc;
 
-    std::vector<int> cont[2];  // resume as is / with a restarted search direction
+    std::vector<int> cont[REZ_NMODE];  // members to resume, by their direction (pcg_rez_kernel)
+    std::vector<std::pair<int, double>> early;  // members stopped early, their next thresholds
     bool desc_changed = false;
     for (int s : rep) {
         Member &M = p->mem[s];
@@ -2631,30 +2656,44 @@ int step_decide(amr_pool *p, std::vector<amr_pool_result> &out)
             }
             desc_changed = true;
         }
+        if (M.early > 0 && M.done && !M.broke) {
+            M.early--;
+            d.thr_fac = stop_factor(M);
+            early.push_back({s, d.thr_fac * M.bb});
+            desc_changed = true;
+        }
         M.broke = 0;
         M.rr_true_prev = rr;
         M.rr_ref = rr;
-        cont[restart ? 1 : 0].push_back(s);
+        cont[restart ? REZ_RESTART : M.unformed ? REZ_FORM : REZ_KEEP].push_back(s);
     }
-    if (cont[0].empty() && cont[1].empty()) return AMR_OK;
-    // resume: r = rt, z = M r (p = z on restart), rz, clear the stop flags
-    std::vector<int2> vc0 = vec_list(p, cont[0]), vc1 = vec_list(p, cont[1]);
-    std::vector<int32_t> sc(cont[0].begin(), cont[0].end());
-    sc.insert(sc.end(), cont[1].begin(), cont[1].end());
+    // resume: r = rt, z = M r, the direction, rz, clear the stop flags
+    std::vector<int2> vc[REZ_NMODE];
+    std::vector<int32_t> sc;
+    size_t nvc = 0;
+    for (int k = 0; k < REZ_NMODE; k++) {
+        vc[k] = vec_list(p, cont[k]);
+        nvc += padded(vc[k]);
+        sc.insert(sc.end(), cont[k].begin(), cont[k].end());
+    }
+    if (sc.empty()) return AMR_OK;
+    for (const auto &e : early)
+        AMR_HIP(hipMemcpyAsync(p->hD[e.first].scal + S_THR, &e.second, sizeof(double), hipMemcpyHostToDevice, st));
+    if (!early.empty())
+        if (int rc = pool_sync(p)) return rc;
     std::vector<int> call(sc.begin(), sc.end());
-    std::vector<int2> ac = agg_list(p, call), cc = cw_list(p, call), pc = vec_list(p, tl_only(p, cont[1]));
-    if (int rc = pool_reserve_lists(p, padded(vc0) + padded(vc1) + padded(sc) + padded(ac) + padded(cc) + padded(pc)))
-        return rc;
+    std::vector<int2> ac = agg_list(p, call), cc = cw_list(p, call), pc = vec_list(p, tl_only(p, cont[REZ_RESTART]));
+    if (int rc = pool_reserve_lists(p, nvc + padded(sc) + padded(ac) + padded(cc) + padded(pc))) return rc;
     Ls.off = 0;
-    const size_t o_vc0 = Ls.push(vc0), o_vc1 = Ls.push(vc1), o_sc = Ls.push(sc);
+    size_t o_vc[REZ_NMODE];
+    for (int k = 0; k < REZ_NMODE; k++) o_vc[k] = Ls.push(vc[k]);
+    const size_t o_sc = Ls.push(sc);
     const size_t o_ac = Ls.push(ac), o_cc = Ls.push(cc), o_pc = Ls.push(pc);
     if (int rc = upload(p, Ls.off, desc_changed || p->desc_dirty)) return rc;
-    if (!vc0.empty())
-        hipLaunchKernelGGL(pcg_rez_kernel, dim3((unsigned)vc0.size()), dim3(WGV), 0, st, p->dD,
-                           Ls.dev_at<int2>(o_vc0), 0);
-    if (!vc1.empty())
-        hipLaunchKernelGGL(pcg_rez_kernel, dim3((unsigned)vc1.size()), dim3(WGV), 0, st, p->dD,
-                           Ls.dev_at<int2>(o_vc1), 1);
+    for (int k = 0; k < REZ_NMODE; k++)
+        if (!vc[k].empty())
+            hipLaunchKernelGGL(pcg_rez_kernel, dim3((unsigned)vc[k].size()), dim3(WGV), 0, st, p->dD,
+                               Ls.dev_at<int2>(o_vc[k]), k);
     launch_tl_fresh(p, Ls, o_ac, (unsigned)ac.size(), o_cc, (unsigned)cc.size(), o_pc, (unsigned)pc.size());
     hipLaunchKernelGGL(pcg_finalize_kernel, dim3((unsigned)sc.size()), dim3(WGV), 0, st, p->dD,
                        Ls.dev_at<int32_t>(o_sc), 2);
@@ -2711,6 +2750,14 @@ int amr_pool_run(amr_pool *p, std::vector<amr_pool_result> &out)
 {
     if (int rc = amr_pool_step_launch(p)) return rc;
     return amr_pool_step_collect(p, out);
+}
+
+extern "C" int amr_test_early_stops(amr_model *m, int n, double rtol)
+{
+    if (!m || n < 0 || (n > 0 && !(rtol > 0.0 && rtol < 1.0))) return AMR_ERR_ARG;
+    m->test_early = n;
+    m->test_early_rtol = rtol;
+    return AMR_OK;
 }
 
 int amr_pool_set_timing(amr_pool *p, int enable, double *ms, int64_t *n)
