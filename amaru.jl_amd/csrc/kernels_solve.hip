@@ -2637,7 +2637,7 @@ int step_decide(amr_pool *p, std::vector<amr_pool_result> &out)
             // tolerance twice, or broke down: finish on the assembled matrix,
             // whose residual decides
             M.mf = false;
-            M.fell_back = M.pc32 ? 1 : 0;
+            M.fell_back = 1;
             restart = true;
         } else if ((M.done && !M.broke && rr > 0.25 * M.rr_true_prev) || (M.broke && ++M.breakdowns > 3)) {
             finish(p, s, out);  // stagnation above both bounds, or repeated breakdown

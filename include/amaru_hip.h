@@ -75,7 +75,9 @@ typedef struct {
     int iterations;     /* PCG iterations performed (inner ones for mixed) */
     int refinements;    /* FP64 residual recomputations (residual replacements) */
     int converged;      /* 1 if rtol (or the rounding floor of the residual) was met */
-    int fallback;       /* mixed: 1 if the solve finished on the FP64 operator */
+    int fallback;       /* 1 if the solve finished on another operator than it began with:
+                           mixed, the FP64 matrix; all-elastic, the assembled FP64 matrix
+                           in place of the matrix-free operator (any precision) */
     double relres;      /* final ||b - K11 x|| / ||b|| evaluated in FP64 */
 } amr_solve_info;
 
@@ -194,7 +196,7 @@ typedef struct {
     int pcg_iterations;  /* PCG iterations of this NR iteration */
     int status;          /* AMR_OK, or the error code of a failed iteration */
     int replacements;    /* FP64 residual recomputations in the linear solve */
-    int fallback;        /* mixed: 1 if the solve finished on the FP64 operator */
+    int fallback;        /* as in amr_solve_info */
 } amr_nr_info;
 
 /* Uex, Fex (ndofs, eq order): essential values and natural loads of the

@@ -69,10 +69,10 @@ def test_refused_stops(amaru, operator, precond, check):
         assert r["replacements"] == n + 1
         # the second refused stop ends the use of the matrix-free operator
         changed = operator == "matrix_free" and n == 2
+        assert r["fallback"] == changed
         if changed:
             assert r["iterations"] <= 2 * r0["iterations"]
         else:
-            assert not r["fallback"]
             assert abs(r["iterations"] - r0["iterations"]) <= 3
         assert np.linalg.norm(U - U0) <= 1e-8 * np.linalg.norm(U0)
     early(dev, 0)
@@ -123,6 +123,7 @@ def test_change_of_operator_in_a_pool(amaru, graphs):
         dev.nr_finish(si)
         gU, gF = dev.stage_get(last=True)
         assert np.array_equal(gU, dU) and np.array_equal(gF, dF)
+    assert [a[2] for a in alone] == [True, True, False, False, False, False]
     for dev, o in devs:
         dev.close()
     pool.close()
