@@ -83,6 +83,7 @@ int amr_pattern_host(amr_model *m);
 
 // Device memory of a model, counted in m->dev_bytes; amr_release gives it back.
 int amr_dalloc(amr_model *m, void **p, size_t bytes);
+hipError_t amr_hip_malloc(amr_model *m, void **p, size_t bytes);
 void amr_release(amr_model *m, void *p);
 
 // Host-built coarse space of the two-level preconditioner (model_build.cpp).
@@ -250,6 +251,9 @@ struct amr_model {
 // later solves stops n times too early, the k-th time (from 1) at rtol^k of
 // |b|, so that the check of the true residual refuses the stop (n = 0: off).
 extern "C" int amr_test_early_stops(amr_model *m, int n, double rtol);
+// For tests: device allocations for models on this thread fail with "out of
+// memory" where they would take the model above that many bytes (< 0: off).
+extern "C" void amr_test_model_bytes(int64_t bytes);
 
 enum { SV_UEX = 0, SV_FEX, SV_U, SV_F, SV_DFEX, SV_R, SV_RC, SV_DUA, SV_DUI, SV_DFIN, SV_DUT, SV_X };
 

@@ -229,14 +229,50 @@ void arena_trim_locked(int device)
     A.blocks.clear();
     A.bytes = 0;
 }
+
+// device bytes a model of this thread may hold (amr_test_model_bytes; < 0: any)
+thread_local int64_t t_model_bytes = -1;
+
+bool over_test_limit(const amr_model *m, size_t bytes)
+{
+    return t_model_bytes >= 0 && m->dev_bytes + (int64_t)bytes > t_model_bytes;
+}
 }  // namespace
+
+extern "C" void amr_test_model_bytes(int64_t bytes) { t_model_bytes = bytes; }
+
+// hipMalloc for a model.  Out of memory, the device's cached blocks are freed
+// first, then the model's matrix-free operator (unless it is solving with it
+// in a pool): it goes on with the assembled matrix.
+hipError_t amr_hip_malloc(amr_model *m, void **p, size_t bytes)
+{
+    auto attempt = [&]() { return over_test_limit(m, bytes) ? hipErrorOutOfMemory : hipMalloc(p, bytes); };
+    auto trim = [&]() {
+        (void)hipGetLastError();
+        std::lock_guard<std::mutex> lk(g_dmem_mu);
+        arena_trim_locked(m->device);
+    };
+    hipError_t e = attempt();
+    if (e == hipErrorOutOfMemory) {
+        trim();
+        e = attempt();
+    }
+    if (e == hipErrorOutOfMemory && m->mf_block && !amr_pool_is_member(m)) {
+        (void)hipStreamSynchronize(m->stream);
+        amr_mf_free(m);
+        trim();
+        e = attempt();
+    }
+    return e;
+}
 
 int amr_dalloc(amr_model *m, void **p, size_t bytes)
 {
     if (bytes == 0) bytes = 1;
     const size_t need = arena_round(bytes);
     const int dev = m->device;
-    {
+    *p = nullptr;
+    if (!over_test_limit(m, need)) {
         std::lock_guard<std::mutex> lk(g_dmem_mu);
         Arena &A = g_arena[dev];
         auto it = A.blocks.lower_bound(need);
@@ -247,8 +283,6 @@ int amr_dalloc(amr_model *m, void **p, size_t bytes)
             A.bytes -= sz;
             g_dmem_live[*p] = {sz, bytes, dev};
             m->dev_bytes += (int64_t)bytes;
-        } else {
-            *p = nullptr;
         }
     }
     if (*p) {
@@ -256,15 +290,7 @@ int amr_dalloc(amr_model *m, void **p, size_t bytes)
         AMR_HIP(hipMemsetAsync(*p, 0, need, m->stream));
         return AMR_OK;
     }
-    hipError_t e = hipMalloc(p, need);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        {
-            std::lock_guard<std::mutex> lk(g_dmem_mu);
-            arena_trim_locked(dev);
-        }
-        e = hipMalloc(p, need);
-    }
+    const hipError_t e = amr_hip_malloc(m, p, need);
     if (e != hipSuccess) {
         *p = nullptr;
         amr_set_error(std::string("hipMalloc of ") + std::to_string(need) + " bytes failed: " + hipGetErrorString(e));
@@ -753,7 +779,7 @@ extern "C" int amr_state_get(amr_model *m, double *st, int committed)
         if (buf) AMR_HIP(hipFree(buf));
         buf = nullptr;
         g_stage_cap[m->device] = 0;
-        AMR_HIP(hipMalloc((void **)&buf, cnt * sizeof(double)));
+        AMR_HIP(amr_hip_malloc(m, (void **)&buf, cnt * sizeof(double)));
         g_stage_cap[m->device] = cnt;
     }
     const unsigned g = (unsigned)((cnt + 255) / 256);

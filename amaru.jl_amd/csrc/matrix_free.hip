@@ -169,7 +169,8 @@ int amr_mf_build(amr_model *m, const double *dNdR_host)
                  o_flag = slice(4);
     const int rc = amr_dalloc(m, (void **)&m->mf_block, off);
     if (rc == AMR_ERR_NOMEM) {
-        // the model still fits without: it iterates on the assembled matrix
+        // the model does without: it iterates on the assembled matrix (so it
+        // does when a later allocation needs the block, amr_hip_malloc)
         (void)hipGetLastError();
         m->mf_block = nullptr;
         return AMR_OK;
@@ -208,8 +209,8 @@ int amr_mf_check(amr_model *m)
     int32_t flag = 0;
     AMR_HIP(hipMemcpyAsync(&flag, m->mf_flag, sizeof flag, hipMemcpyDeviceToHost, m->stream));
     AMR_HIP(hipStreamSynchronize(m->stream));
-    m->mf_ok = flag == 0;
-    if (!m->mf_ok) amr_mf_free(m);
+    if (flag == 0) m->mf_ok = true;
+    else amr_mf_free(m);
     return AMR_OK;
 }
 
@@ -217,4 +218,5 @@ void amr_mf_free(amr_model *m)
 {
     amr_release(m, m->mf_block);
     m->mf_block = nullptr;
+    m->mf_ok = false;
 }

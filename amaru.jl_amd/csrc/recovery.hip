@@ -381,7 +381,7 @@ template <typename T>
 int alloc(amr_model *m, T **p, size_t n, int64_t &bytes)
 {
     if (n == 0) n = 1;
-    hipError_t e = hipMalloc((void **)p, n * sizeof(T));
+    const hipError_t e = amr_hip_malloc(m, (void **)p, n * sizeof(T));
     if (e != hipSuccess) {
         *p = nullptr;
         amr_set_error(std::string("hipMalloc of ") + std::to_string(n * sizeof(T)) + " bytes failed: " +
