@@ -481,10 +481,12 @@ def estimate_device_bytes(model):
     per_node = 888
     per_elem = 4 * nn + 4 + 72 * nn * nn + 24 * nn + 4 + 4 * nn + 224 * nips + 4 * nn * nn
     per_blk = 4 + 8 + 72 + 36 + 9
-    # matrix-free operator: geometry per IP, node ids and products per element
-    # node, in groups of 16 elements
-    grp = (ne + 15) // 16
-    mf = grp * (-(-nips // 4) * 4608 + -(-nn // 4) * 1792 + 256) + 4 * ne * nn + 32 * nnodes + 32768 if ne else 0
+    # matrix-free operator (models whose materials are all elastic): geometry
+    # per IP, node ids and products per element node, in groups of 16 elements
+    mf = 0
+    if ne and all(m.kind == _lib.AMR_MAT_LE for m in model.mats):
+        grp = (ne + 15) // 16
+        mf = grp * (-(-nips // 4) * 4608 + -(-nn // 4) * 1792 + 256) + 4 * ne * nn + 32 * nnodes + 32768
     # + the padding of the 32 vector slices (to 64 entries each)
     return int(per_node * nnodes + per_elem * ne + per_blk * (nblk + 64) + mf + 46080 * 8 + 4096 + 24 * 64 * 8 + 8 * 64 * 4)
 

@@ -328,6 +328,22 @@ def test_device_bytes_estimate_is_monotone(amaru):
     assert math.isfinite(prev)
 
 
+@pytest.mark.parametrize("shape,nips", [("HEX8", 8), ("HEX20", 8), ("HEX20", 27), ("TET10", 4)])
+def test_device_bytes_estimate_counts_the_elastic_operator_for_elastic_models(amaru, shape, nips):
+    """Only all-elastic models hold the matrix-free operator's element data:
+    72 bytes per IP and more, in groups of 16 elements."""
+    from amaru_amd import pool as P
+    mesh = amaru.Mesh(amaru.Block([[0, 0, 0], [1, 1, 1]], nx=5, ny=4, nz=3, cellshape=shape))
+    mesh.tags = np.where(np.arange(mesh.ne) < 7, "b", "a").astype(object)
+    le, vm = amaru.LinearElastic(E=1e9, nu=0.3), amaru.VonMises(E=1e9, nu=0.3, fy=1e6, H=0.0)
+
+    def est(a, b):
+        return P.estimate_device_bytes(amaru.FEModel(mesh, [("a", amaru.MechSolid, a), ("b", amaru.MechSolid, b)],
+                                                     nips=nips))
+    assert est(vm, vm) == est(le, vm) == est(vm, le)
+    assert est(le, le) - est(vm, vm) >= 72 * nips * mesh.ne
+
+
 def test_server_counts_unfreed_models_in_admission(amaru, monkeypatch):
     """Finished models are freed at idle points; until then their bytes
     count against the budget, so admitted plus unfreed bytes never exceed
