@@ -1041,8 +1041,10 @@ __global__ void __launch_bounds__(WGV) pcg_update_kernel(const SegDesc *__restri
     const int pi = (iters - 1) & 1;
     auto *__restrict__ x = glw(d.x);
     auto *__restrict__ r = glw(d.r);
-    auto *__restrict__ z = glw(d.z);
-    auto *__restrict__ p = glw(d.p);
+    // (no __restrict__: where the direction is formed, z and p are read through
+    // zs and written here)
+    auto *z = glw(d.z);
+    auto *p = glw(d.p);
     const auto *__restrict__ q = gl(d.q);
     const double beta = FUSE ? (double)glw(d.scal)[S_BETA] : 0.0;
     const double rzp0 = glw(d.scal)[S_RZP0], rzp1 = glw(d.scal)[S_RZP1];
