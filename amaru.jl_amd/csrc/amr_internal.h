@@ -242,8 +242,8 @@ struct amr_model {
     int32_t *mf_conn = nullptr, *mf_src = nullptr, *mf_rec = nullptr, *mf_flag = nullptr;
     char *mf_block = nullptr;       // the arrays above are slices of it
     std::vector<double> mf_tab_h;   // host copy of mf_tab while it is uploaded
-    // set by tests only (amr_test_early_stops)
-    int test_early = 0;
+    // set by tests only (amr_test_early_stops, amr_test_limits)
+    int test_early = 0, test_tiles = 0, test_chunks = 0;
     double test_early_rtol = 0.0;
 };
 
@@ -251,6 +251,10 @@ struct amr_model {
 // later solves stops n times too early, the k-th time (from 1) at rtol^k of
 // |b|, so that the check of the true residual refuses the stop (n = 0: off).
 extern "C" int amr_test_early_stops(amr_model *m, int n, double rtol);
+// For tests: at most that many tiles of the matrix-free operator, and chunks of
+// a coarse space built afterwards (where its aggregates allow), so that a small
+// model takes the passes of a large one (0: the usual limits).
+extern "C" int amr_test_limits(amr_model *m, int tiles, int chunks);
 // For tests: device allocations for models on this thread fail with "out of
 // memory" where they would take the model above that many bytes (< 0: off).
 extern "C" void amr_test_model_bytes(int64_t bytes);

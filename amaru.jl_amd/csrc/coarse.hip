@@ -427,6 +427,7 @@ int build(amr_model *m)
     if (int rc = dev_upload(m, &m->c_aggnodes, C.aggnodes)) return rc;
     // chunks of at most 256 k nodes (k passes of a workgroup), the smallest k
     // that keeps the chunks' partials within their 1,024 slots
+    const int32_t slots = m->test_chunks ? m->test_chunks : 1024;
     for (int64_t k = 1;; k++) {
         C.chunk.clear();
         C.aggch.assign(1, 0);
@@ -436,7 +437,7 @@ int build(amr_model *m)
                                {(int32_t)b, (int32_t)std::min<int64_t>(C.aggptr[a + 1], b + 256 * k), a, 0});
             C.aggch.push_back((int32_t)(C.chunk.size() / 4));
         }
-        if (C.aggch.back() <= 1024 || 256 * k >= n) break;
+        if (C.aggch.back() <= slots || 256 * k >= n) break;
     }
     m->nchunk = C.aggch.back();
     if (int rc = dev_upload(m, &m->c_chunk, C.chunk)) return rc;

@@ -1572,8 +1572,9 @@ MfGeom mf_geom(const amr_model *m)
 {
     MfGeom g;
     g.W = m->nips == 27 ? (m->mf_ngrp < 1024 ? 4 : 1) : m->nips == 8 ? (m->mf_ngrp < 256 ? 2 : 1) : 1;
-    const int64_t ng = 4 / g.W;
-    g.G = (int)std::max<int64_t>(1, (m->mf_ngrp + ng * MAX_GR - 1) / (ng * MAX_GR));
+    if (m->test_tiles) g.W = 1;  // (a shared group's waves take one group only)
+    const int64_t ng = 4 / g.W, most = m->test_tiles ? m->test_tiles : MAX_GR;
+    g.G = (int)std::max<int64_t>(1, (m->mf_ngrp + ng * most - 1) / (ng * most));
     g.ntiles = (int)((m->mf_ngrp + ng * g.G - 1) / (ng * g.G));
     return g;
 }
@@ -2759,6 +2760,14 @@ extern "C" int amr_test_early_stops(amr_model *m, int n, double rtol)
     if (!m || n < 0 || (n > 0 && !(rtol > 0.0 && rtol < 1.0))) return AMR_ERR_ARG;
     m->test_early = n;
     m->test_early_rtol = rtol;
+    return AMR_OK;
+}
+
+extern "C" int amr_test_limits(amr_model *m, int tiles, int chunks)
+{
+    if (!m || tiles < 0 || tiles > MAX_GR || chunks < 0 || chunks > MAX_GV) return AMR_ERR_ARG;
+    m->test_tiles = tiles;
+    m->test_chunks = chunks;
     return AMR_OK;
 }
 

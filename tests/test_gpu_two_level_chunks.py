@@ -8,12 +8,21 @@ Drucker-Prager material keeps the assembled matrix, where the update kernel
 works by chunks; the elastic one takes the matrix-free operator, where it
 does not.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 from oracle import HEX8 as O8, fem
 
 pytestmark = pytest.mark.gpu
+
+
+def limits(dev, chunks):
+    from amaru_amd import _lib
+    f = _lib.lib().amr_test_limits
+    f.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int]
+    _lib.check(f(dev.handle, 0, chunks))
 
 
 @pytest.mark.parametrize("plastic", [True, False])
@@ -43,8 +52,12 @@ def test_chunks_match_direct(amaru, plastic, target, precision):
     dev.close()
 
 
-@pytest.mark.parametrize("target", [3, 64, 256, 257, 1100, 100000])
-def test_restrictions_agree(amaru, target):
+# chunks: the slots of their partials (0: 1,024); fewer slots than the
+# aggregates have chunks of 256 nodes make chunks of 512 (1100, 8), 768 and
+# 2,816 nodes, which a workgroup takes in several passes
+@pytest.mark.parametrize("target,chunks", [(3, 0), (64, 0), (256, 0), (257, 0), (1100, 0), (100000, 0), (1100, 8),
+                                           (1100, 4), (100000, 4), (100000, 1)])
+def test_restrictions_agree(amaru, target, chunks):
     """The restriction's own kernel (elastic models) against the chunks of the
     update kernel (Drucker-Prager, not yet plastic: the same K), with
     aggregates below, at and above a workgroup's 256 nodes and, at the last,
@@ -61,6 +74,7 @@ def test_restrictions_agree(amaru, target):
         model.configure_dofs(bcs)
         U, F = model.bc_vals(bcs)
         dev = am.DeviceModel(model)
+        limits(dev, chunks)
         dev.set_coarse(target)
         dev.assemble()
         r = dev.solve_system(U, F, rtol=1e-10, precond="two_level")
