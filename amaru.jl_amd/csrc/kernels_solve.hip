@@ -1555,15 +1555,18 @@ Geom model_geom(const amr_model *m)
 }
 
 // Tiles of the matrix-free operator.  With few groups the waves of a
-// workgroup share a group where its IP slots can be divided: such a launch is
-// bound by one wave's chain of matrix instructions, not by throughput.  Four
-// waves a group for 27 IPs below 1,024 groups (a wave per SIMD; HEX20 17x19x15,
-// 303 groups: 12.3 us with one wave per group, 10.3 with four), two for the hex
-// rules with 8 IPs below 256 (HEX20 64x7x8, 224 groups: 7.2 against 6.2 us;
-// HEX8 57x15x13, 695 groups: 3% slower passes with two).  From there on a wave
-// takes a group of its own, G groups in turn only where the p.q partials would
-// not fit otherwise (two groups a wave made the 40^3 HEX20 block no faster and
-// the TET10 49x12x13 box 10% slower).
+// workgroup share a group where its IP slots can be divided (four waves a group
+// for 27 IPs, two for the hex rules with 8): such a launch is bound by one
+// wave's chain of matrix instructions, not by throughput.  The line is at two
+// groups per CU, 512.  Up to there all workgroups run at once, two per CU with
+// four waves a group (65 KB of LDS each), one with two; the next group starts
+// a second round.  Launches between events, one wave a group against shared,
+// at 512 and 529 groups: HEX20 with 27 IPs 15.3 / 13.8 and 15.3 / 17.7 us, with
+// 8 IPs 10.8 / 10.0 and 11.0 / 11.4, HEX8 8.31 / 8.12 and 8.26 / 8.50; at 46
+// and 938 groups with 27 IPs 13.7 / 9.9 and 15.4 / 21.3.  Above, a wave takes
+// a group of its own, G groups in turn only where the p.q partials would not
+// fit otherwise (two groups a wave made the 40^3 HEX20 block no faster and the
+// TET10 49x12x13 box 10% slower).
 struct MfGeom {
     int W, G, ntiles;
 };
@@ -1571,7 +1574,7 @@ struct MfGeom {
 MfGeom mf_geom(const amr_model *m)
 {
     MfGeom g;
-    g.W = m->nips == 27 ? (m->mf_ngrp < 1024 ? 4 : 1) : m->nips == 8 ? (m->mf_ngrp < 256 ? 2 : 1) : 1;
+    g.W = m->mf_ngrp > 2 * (int64_t)m->ncu ? 1 : m->nips == 27 ? 4 : m->nips == 8 ? 2 : 1;
     if (m->test_tiles) g.W = 1;  // (a shared group's waves take one group only)
     const int64_t ng = 4 / g.W, most = m->test_tiles ? m->test_tiles : MAX_GR;
     g.G = (int)std::max<int64_t>(1, (m->mf_ngrp + ng * most - 1) / (ng * most));

@@ -57,10 +57,11 @@ def close(a, b):
     return np.linalg.norm(a - b) <= 1e-8 * np.linalg.norm(b)
 
 
-# elements: one, around a group (16) and a tile (64), and enough groups for a
-# wave each (from 256 groups; with 27 IPs from 1,024)
-SIZES = {"HEX8": [(2, 1, 1), (5, 3, 1), (4, 4, 1), (17, 1, 1), (9, 7, 1), (4, 4, 4), (13, 5, 1), (33, 32, 32)],
-         "HEX20": [(2, 1, 1), (5, 3, 1), (17, 1, 1), (13, 5, 1), (26, 26, 25)],
+# elements: one, around a group (16) and a tile (64), and around and above the
+# 512 groups up to which waves share a group
+SIZES = {"HEX8": [(2, 1, 1), (5, 3, 1), (4, 4, 1), (17, 1, 1), (9, 7, 1), (4, 4, 4), (13, 5, 1), (16, 16, 32), (17, 22, 22),
+                  (33, 32, 32)],
+         "HEX20": [(2, 1, 1), (5, 3, 1), (17, 1, 1), (13, 5, 1), (16, 16, 32), (17, 22, 22), (26, 26, 25)],
          "TET10": [(2, 1, 1), (3, 1, 1), (11, 1, 1), (4, 3, 2), (19, 13, 11)]}
 
 
