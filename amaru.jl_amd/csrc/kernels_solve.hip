@@ -52,17 +52,22 @@ constexpr int MAX_GR = 8192, MAX_GV = 1024;
 
 // scalar and control slots of one model: S_NSCAL doubles, then C_NCTL ints
 // S_RZP0/1: r.z published per parity slot (the sum of that slot's partials)
-// S_BETA: the running iteration's beta (matrix-free members)
+// S_BETA: the running iteration's beta (members whose operator forms the direction)
 enum { S_RZ = 0, S_RR, S_BB, S_THR, S_KX, S_RES, S_ERRN, S_ERRD, S_GAP, S_RZP0, S_RZP1, S_BETA, S_NSCAL = 16 };
 __device__ inline int rz_pub(int slot) { return slot ? S_RZP1 : S_RZP0; }
 // C_DONE is read by every workgroup at kernel entry and written only where
 // all workgroups of the model in the running launch agree on it
-// (breakdown); the convergence test writes C_STOP, which the next SpMV
-// promotes to C_DONE, so no workgroup ever sees a flag raised during its
-// own launch.  C_ITERS is advanced by the SpMV's first tile and read by the
-// kernels after it.  C_PREV is the number of completed iterations, advanced
-// by the update kernel: the matrix-free operator's tiles read it (one of them
-// writes C_ITERS in the same launch).
+// (breakdown); the convergence test writes C_STOP, which the next operator
+// launch promotes to C_DONE.  Where pcg_dir_kernel tests, it reads no C_STOP,
+// so none of its workgroups sees a flag of its own launch.  Where the operator
+// forms the direction, its first tile tests: later tiles of that launch may
+// see C_STOP and leave, earlier ones work on; either is right, since the
+// update kernel reads C_STOP first, uses nothing of a stopped iteration and
+// promotes the flag itself.  The direction is not stored then (REZ_FORM).
+// C_ITERS is advanced by the operator's first tile and read by the kernels
+// after it.  C_PREV is the number of completed iterations, advanced by the
+// update kernel: the tiles of an operator that forms the direction read it
+// (one of them writes C_ITERS in the same launch).
 enum { C_DONE = 0, C_ITERS, C_BREAK, C_NAN, C_STOP, C_PREV, C_NCTL = 16 };
 constexpr int SEG_DBL = 32;  // doubles per model in a pool's scalar array
 static_assert(S_NSCAL + C_NCTL / 2 <= SEG_DBL, "scalar block");
@@ -502,9 +507,6 @@ __device__ inline double *tile_dbl(char *sm, int R, int j)
     return (double *)(sm + off) + (int64_t)j * pow2ceil(R);
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on
-// XCD b % 8).  Entry t(b) gives each XCD one contiguous run of the work
-// list, so the slice of x a run of row tiles gathers stays in that XCD's L2.
 // Entry i of a launch's work list.  A step with one member needs none: the
 // launch passes a null list and that member's descriptor, which takes one
 // dependent load off the start of every workgroup (a pass through the kernels
@@ -518,11 +520,14 @@ __device__ inline int2 list_entry(const int2 *__restrict__ l, int64_t i)
 // their first loads together with the control words and only then test them,
 // and address past-the-end operands clamped instead of under a branch.  On
 // small models a wave of these kernels waits for memory three quarters of its
-// time, about 0.45 us per dependent load: with this, DPP reductions and no
-// work list, an iteration of the HEX8 20x4x4 model takes 12.0 us instead of
-// 14.6, of the HEX20 64x7x8 one 14.9 us instead of 18.0.
+// time, about 0.45 us per dependent load: this, DPP reductions and no work
+// list together took an iteration of the HEX8 20x4x4 model from 14.6 to 12.0
+// us, of the HEX20 64x7x8 one from 18.0 to 14.9.
 #define AMR_ISSUED() asm volatile("" ::: "memory")
 
+// Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on
+// XCD b % 8).  Entry t(b) gives each XCD one contiguous run of the work
+// list, so the slice of x a run of row tiles gathers stays in that XCD's L2.
 __device__ inline int64_t xcd_tile(int64_t b, int64_t G)
 {
     const int64_t x = b & 7, i = b >> 3, q = G >> 3, rm = G & 7;
@@ -754,15 +759,18 @@ __global__ void __launch_bounds__(WGS) pcg_spmv_kernel(const SegDesc *__restrict
 // gather costs less than a kernel of its own; pcg_update stores it.  The
 // first tile then does pcg_dir_kernel's bookkeeping.
 //
-// Bound: FP64 matrix cores (HEX20 with 27 IPs: 630 v_mfma_f64_4x4x4 per group,
-// 16 cycles each: 16 us for the 64,000 elements of a 40^3 block) plus 72 B per
-// IP of geometry.  The 4x4x4 form is used because its operand and result
-// lanes agree (no exchange) and its rows need no padding to 16; measured
-// alone it reaches 68 TFLOP/s here against 43 for 16x16x4.  On the 40^3 HEX20
-// block: 33.6 us a launch, where the SpMV on the assembled matrix takes 142 us
-// (FP32 values) or 235 us (FP64); HEX20 17x19x15: 14.5 against 20.7 us; HEX8
-// 83x21x20: 11.8 against 12.5 us (FP32) and 23 (FP64), TET10 49x12x13: 9.8
-// against 23.4 and 33.7 us.
+// Bound on the 40^3 HEX20 block (27 IPs, 64,000 elements) by memory: 35 us a
+// launch, in which 144 MB are read (72 B of geometry per IP, most of it) and
+// 31 MB written past the L2, 5.0 TB/s, the rate of a 1 GiB copy; the matrix
+// cores are busy 55% of its cycles (630 v_mfma_f64_4x4x4 per group, 16 cycles
+// each), without LDS bank conflicts.  In small models by one wave's chain (see
+// mf_geom).  The 4x4x4 form is used because its operand and result lanes agree
+// (no exchange) and its rows need no padding to 16; measured alone it reaches
+// 68 TFLOP/s here against 43 for 16x16x4.  Medians of a kernel trace, and of
+// the SpMV on the assembled matrix with FP32 and with FP64 values: the block 35
+// us against 142 and 235; HEX20 17x19x15 10.9 against 15.8 and 20.9; HEX20
+// 64x7x8 with 8 IPs 6.2 against 16.1 and 21.2; HEX8 83x21x20 9.2 against 12.8
+// and 18.2; TET10 49x12x13 10.3 against 22.6 and 33.3 us.
 template <int NN, int NQ>
 struct MfShape {
     static constexpr int NS = (NN + 3) / 4, KS = (NQ + 3) / 4, HALF = KS * 3 * NS * 16;
@@ -882,7 +890,6 @@ __global__ void __launch_bounds__(256, 2) pcg_mf_kernel(const SegDesc *__restric
         if (W == 1 && grp >= d.ngrp) break;  // (a shared group's waves meet at a barrier; mfG is 1 there)
         if (W == 1 && w > 0) {
             load_nodes(grp);
-            if (AHEAD) load_geo(grp, 0);
             gather();
         }
         // the waves of a shared group each gathered some of its nodes (the
@@ -2352,8 +2359,8 @@ int amr_pool_step_launch(amr_pool *p)
     // an assembled matrix, and two-level on an assembled matrix (by chunks of
     // their aggregates); restrictions of the matrix-free two-level members;
     // direction kernels for the one-level members that have one in every
-    // iteration (vd), for all of them in the step's last one (vl), and for
-    // the two-level members (vt)
+    // iteration (V_D), for all of them in the step's last one (V_L), and for
+    // the two-level members (V_T)
     enum { V_M, V_A, V_AF, V_AT, V_RS, V_D, V_L, V_T, V_CW, NV };
     std::vector<int> sv[NV];
     for (int s : act) {

@@ -4,9 +4,8 @@
 // instead of the assembled matrix.
 //
 // What it reads per element is 72 B per IP (HEX20 with 27 IPs: 1.9 KB, HEX8
-// 0.6 KB, TET10 0.3 KB) against 76-82 B per 3x3 block of the assembled matrix
-// (HEX20 about 18 KB of blocks per element), so the operator is bound by the
-// FP64 matrix cores and no longer by the matrix in HBM.
+// 0.6 KB, TET10 0.3 KB) against 38 to 76 B per 3x3 block of the assembled matrix
+// (HEX20: 9 to 18 KB of blocks per element).
 //
 // Layout.  Elements are taken in groups of 16, one wave per group.  Lane l =
 // 16 g + c of a group holds, of element 16 grp + c, the nodes 4 s + g (slot
