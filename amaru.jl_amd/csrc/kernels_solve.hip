@@ -1567,7 +1567,7 @@ Geom model_geom(const amr_model *m)
 // wave's chain of matrix instructions, not by throughput.  The line is at two
 // groups per CU, 512.  Up to there all workgroups run at once, two per CU with
 // four waves a group (65 KB of LDS each), one with two; a workgroup more
-// waits until one has ended.  Launches between events, one wave a group against shared,
+// waits for a place, or shares a CU with another.  Launches between events, one wave a group against shared,
 // at 512 and 529 groups: HEX20 with 27 IPs 15.3 / 13.8 and 15.3 / 17.7 us, with
 // 8 IPs 10.8 / 10.0 and 11.0 / 11.4, HEX8 8.31 / 8.12 and 8.26 / 8.50; at 46
 // and 938 groups with 27 IPs 13.7 / 9.9 and 15.4 / 21.3.  Above, a wave takes
